@@ -1,0 +1,54 @@
+/*
+ * prompt_ops.h -- entry points behind Qwen2Runner's prompt pass (libnanoserve_amd.so), called by
+ * nanoserve_amd/ops.py. Conventions of include/nanoserve_decode.h: caller-allocated device
+ * memory, bf16 tensors as void*, asynchronous on `stream`, no allocation, capturable; 0 on
+ * success, -2 for rejected arguments (checked before any HIP call), else the hipError_t.
+ */
+#ifndef NANOSERVE_PROMPT_OPS_H
+#define NANOSERVE_PROMPT_OPS_H
+
+#include <stddef.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/*
+ * Bias + RoPE + KV-cache append of T prompt tokens at positions pos0 .. pos0 + T - 1 (the
+ * reference does these with PyTorch ops and ns_rope, python/nanoserve/qwen.py:119-122, 147-151).
+ * qkv [T][Hq + 2 Hk][D]: every element gets bf16_rne(qkv + bias) (bias NULL: no add) and the q
+ * and k heads are rotated as by ns_rope. q heads are updated in place; with k_cache / v_cache
+ * [Hk][max_len][D] the k and v heads go to rows pos0 .. of the caches (qkv keeps their old
+ * values), without them (both NULL) they are updated in place.
+ * -2 for D % 16 != 0, D > 512, sizes <= 0, pos0 < 0, one cache without the other, rows past
+ * max_len, NULL or misaligned pointers (qkv, bias and the caches 16-byte aligned).
+ */
+int ns_prompt_qkv(void* qkv, const void* bias, const void* inv_freq, void* k_cache,
+                  void* v_cache, int T, int Hq, int Hk, int D, int pos0, int max_len,
+                  void* stream);
+
+/*
+ * Bytes of workspace ns_prompt_attention uses for these sizes (fp32 partials of the splits over
+ * the keys); 0 when the queries alone fill the GPU and nothing is split, or for invalid sizes.
+ */
+size_t ns_prompt_attention_workspace(int T, int Hq, int Hk, int pos0);
+
+/*
+ * Causal grouped-query attention of T prompt tokens at positions pos0 .. pos0 + T - 1 (the
+ * reference uses PyTorch SDPA, python/nanoserve/qwen.py:124-133). Query t attends over keys
+ * 0 .. pos0 + t. q: token stride q_stride, heads [Hq][128] contiguous; k, v: key j of kv head g
+ * at g * kv_head_stride + j * kv_stride (strides in elements), 128 values each; out
+ * [T][Hq * 128] bf16. Products of the bf16 operands and all sums in fp32, softmax in fp32, the
+ * probabilities to 16 significant bits (two bf16 terms).
+ * -2 for Hq % Hk != 0, sizes <= 0, pos0 < 0, strides not a multiple of 8 or rows that reach
+ * 2 GiB, NULL or pointers that are not 16-byte aligned, work_bytes too small.
+ */
+int ns_prompt_attention(const void* q, long long q_stride, const void* k, const void* v,
+                        long long kv_stride, long long kv_head_stride, void* out, void* work,
+                        size_t work_bytes, int T, int Hq, int Hk, int pos0, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* NANOSERVE_PROMPT_OPS_H */

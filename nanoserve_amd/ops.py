@@ -50,7 +50,14 @@ SIGNATURES["ns_probe_read"] = [_VP, _SZ, _VP, _I32, _I32, _I32, _VP]
 SIGNATURES["ns_probe_empty"] = [_I32, _I32, _VP]
 SIGNATURES["ns_probe_linear_loop"] = [_VP] * 7 + [_I32, _I32, _VP]
 RESTYPES = {"ns_decode_attention_workspace": _SZ, "ns_w4_gptq_workspace": _SZ,
-            "ns_w4_linear_workspace": _SZ}
+            "ns_w4_linear_workspace": _SZ, "ns_prompt_attention_workspace": _SZ}
+# Entry points of this package's own callers (csrc/prompt_ops.h), not part of the public ABI.
+INTERNAL_SIGNATURES = {
+    "ns_prompt_qkv": [_VP] * 5 + [_I32] * 6 + [_VP],
+    "ns_prompt_attention_workspace": [_I32] * 4,
+    "ns_prompt_attention": [_VP, _I64, _VP, _VP, _I64, _I64, _VP, _VP, _SZ, _I32, _I32, _I32, _I32,
+                            _VP],
+}
 
 
 if hasattr(torch._C, "_cuda_getCurrentRawStream"):
@@ -92,7 +99,7 @@ class Kernels:
             raise OSError(f"{path} not found: build it with `python -m nanoserve_amd.build` "
                           "(there is no CPU fallback)")
         self.lib = ctypes.CDLL(path)
-        for name, args in SIGNATURES.items():
+        for name, args in {**SIGNATURES, **INTERNAL_SIGNATURES}.items():
             fn = getattr(self.lib, name)
             fn.argtypes = args
             fn.restype = RESTYPES.get(name, ctypes.c_int)
@@ -471,6 +478,74 @@ class Kernels:
         rc = self.lib.ns_bf16_gemv(ptr(x), ptr(res), ptr(r), ptr(norm_w), eps, W.data_ptr(),
                                    out.data_ptr(), N, K, self._stream())
         self._check(rc, "ns_bf16_gemv")
+        return out
+
+    # ------------------------------------------------------------------ prompt-pass attention
+    def prompt_qkv(self, qkv, bias, inv_freq, n_heads, n_kv_heads, head_dim, pos0, k_cache=None,
+                   v_cache=None):
+        """T prompt tokens at positions pos0 ..: bias add + RoPE of the fused projection output
+        qkv [T, (Hq + 2Hk) * D], q heads in place, k and v heads into rows pos0 .. of one layer's
+        k_cache / v_cache [Hk, max_len, D], or in place without them (csrc/prompt_ops.h). The
+        reference does this with PyTorch ops and ns_rope (qwen.py:119-122, 147-151)."""
+        _require_gpu_tensor(qkv, "qkv", torch.bfloat16)
+        _require_gpu_tensor(inv_freq, "inv_freq", torch.float32)
+        if qkv.dim() != 2 or not qkv.is_contiguous() or (
+                qkv.shape[1] != (n_heads + 2 * n_kv_heads) * head_dim):
+            raise ValueError("qkv must be a contiguous [T, (Hq + 2Hk) * D] tensor")
+        if inv_freq.numel() != head_dim // 2 or not inv_freq.is_contiguous():
+            raise ValueError("inv_freq must be contiguous with head_dim / 2 elements")
+        if bias is not None:
+            _require_gpu_tensor(bias, "bias", torch.bfloat16)
+            if bias.numel() != qkv.shape[1] or not bias.is_contiguous():
+                raise ValueError("bias must be contiguous with one value per column of qkv")
+        for t, n in ((k_cache, "k_cache"), (v_cache, "v_cache")):
+            if t is not None:
+                _require_gpu_tensor(t, n, torch.bfloat16)
+                if not t.is_contiguous() or t.shape[0] != n_kv_heads or t.shape[2] != head_dim:
+                    raise ValueError(f"{n} must be a contiguous [Hk, max_len, D] tensor")
+        if k_cache is not None and v_cache is not None and k_cache.shape != v_cache.shape:
+            raise ValueError("k_cache and v_cache must have the same shape")
+
+        def ptr(t):
+            return None if t is None else t.data_ptr()
+
+        rc = self.lib.ns_prompt_qkv(qkv.data_ptr(), ptr(bias), inv_freq.data_ptr(), ptr(k_cache),
+                                    ptr(v_cache), qkv.shape[0], n_heads, n_kv_heads, head_dim,
+                                    pos0, 0 if k_cache is None else k_cache.shape[1],
+                                    self._stream())
+        self._check(rc, "ns_prompt_qkv")
+
+    def prompt_attention_workspace(self, T, n_heads, n_kv_heads, pos0, device=None):
+        """A uint8 device tensor of the workspace prompt_attention uses for these sizes, or None.
+        Launches that may overlap in time need workspaces of their own."""
+        n = int(self.lib.ns_prompt_attention_workspace(T, n_heads, n_kv_heads, pos0))
+        return torch.empty(n, dtype=torch.uint8, device=device or "cuda") if n else None
+
+    def prompt_attention(self, q, k, v, n_heads, pos0, work=None, out=None):
+        """Causal grouped-query attention, head size 128: q [T, >= Hq * 128] (rows may be strided)
+        at positions pos0 .. pos0 + T - 1 over k, v [Hk, >= pos0 + T, 128] (the same strides, last
+        dimension contiguous: a layer's cache, or heads of the projection's rows); returns
+        [T, Hq * 128] bf16. Reference: PyTorch SDPA (qwen.py:124-133)."""
+        for t, n in ((q, "q"), (k, "k"), (v, "v")):
+            _require_gpu_tensor(t, n, torch.bfloat16)
+        T, Hk = q.shape[0], k.shape[0]
+        if q.stride(1) != 1 or q.shape[1] < n_heads * 128:
+            raise ValueError("q rows must be contiguous and hold n_heads * 128 values")
+        if k.shape != v.shape or k.stride() != v.stride() or k.shape[2] != 128 or k.stride(2) != 1:
+            raise ValueError("k and v must be alike, with contiguous rows of 128 values")
+        if k.shape[1] < pos0 + T:
+            raise ValueError(f"k and v must hold {pos0 + T} rows")
+        if out is None:
+            out = torch.empty((T, n_heads * 128), dtype=torch.bfloat16, device=q.device)
+        else:
+            _require_gpu_tensor(out, "out", torch.bfloat16)
+            if tuple(out.shape) != (T, n_heads * 128) or not out.is_contiguous():
+                raise ValueError(f"out must be a contiguous [{T}, {n_heads * 128}] tensor")
+        rc = self.lib.ns_prompt_attention(
+            q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k.stride(1), k.stride(0),
+            out.data_ptr(), None if work is None else work.data_ptr(),
+            0 if work is None else work.numel(), T, n_heads, Hk, pos0, self._stream())
+        self._check(rc, "ns_prompt_attention")
         return out
 
     # ------------------------------------------------------------------ packed tile format

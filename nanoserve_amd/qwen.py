@@ -22,9 +22,9 @@ with the residual add + RMSNorm fused into their activation load, SwiGLU fused i
 gate/up GEMV's output; the down GEMV), ns_decode_qkv_attention (bias + RoPE + KV append +
 grouped-query attention over the cache, splits left unmerged) and ns_w4_gemv_decode_attn
 (the o GEMV, merging the attention's splits while loading its activation). The gate/up weight rows are stored interleaved in blocks of 8
-(``interleave_gate_up``) so that a gate row and its up row land in the same 16-row group. The prompt pass (T > 1) uses ns_w4_linear (GEMM for T > 8) and ns_w4_linear_swiglu, ns_rope,
-ns_rmsnorm, and PyTorch attention for the prompt's causal attention (the fused bf16 SDPA kernel
-for a prompt from position 0, fp32 SDPA over cached positions); after
+(``interleave_gate_up``) so that a gate row and its up row land in the same 16-row group. The prompt pass (T > 1) uses ns_w4_linear (GEMM for T > 8) and ns_w4_linear_swiglu,
+ns_rmsnorm, ns_prompt_qkv (bias + RoPE + KV append) and ns_prompt_attention (causal attention on
+matrix cores; PyTorch SDPA for head sizes other than 128); after
 ``pack_prefill`` prompts of more than 16 tokens run the packed-format GEMMs instead
 (ns_w4_linear_packed, ns_w4_linear_packed_swiglu).
 
@@ -292,13 +292,6 @@ class Qwen2Runner:
         self.merge_in_o = max_len <= 16 * ATTN_SPLIT_ROWS
         self.graph = None
 
-    def _store_kv(self, li, k, v, pos0):
-        """Write the prompt's k and v rows ([T, kv_heads * D] each) into cache rows
-        pos0 .. pos0 + T - 1 of layer li (cache layout [kv_heads][max_len][D])."""
-        D, T = self.shape.head_dim, k.shape[0]
-        for cache, rows in ((self.cache_k, k), (self.cache_v, v)):
-            cache[li].narrow(1, pos0, T).copy_(rows.unflatten(1, (-1, D)).permute(1, 0, 2))
-
     # ------------------------------------------------------------------ one-token decode step
     def _decode_body(self):
         """One decode step on self.tok / self.pos (device tensors) into self.logits. Launches
@@ -403,9 +396,17 @@ class Qwen2Runner:
             self.packed.append(P)
         return self
 
+    def _prompt_attention_kernel_ok(self, T, pos0):
+        """Whether ns_prompt_attention takes this chunk: head size 128, and its 32-bit offsets
+        (keys in the cache rows or, without a cache, in the projection's rows; row tiles)."""
+        s = self.shape
+        return (s.head_dim == 128 and (pos0 + T + 128) * s.qkv_rows * 2 < 1 << 31
+                and T * (s.heads // s.kv_heads) < 1 << 23)
+
     def _prompt_attention(self, q, k, v, pos0, li):
         """Causal attention of T query tokens at positions pos0 .. pos0+T-1 over cache / prompt
-        keys (PyTorch), returned as bf16 [T, Hq*D]. A prompt from position 0 runs the fused SDPA
+        keys (PyTorch) where ns_prompt_attention does not apply, returned as bf16 [T, Hq*D]. A
+        prompt from position 0 runs the fused SDPA
         kernel (flash or memory-efficient backend: fp32 scores, softmax and sums) on the bf16
         q / k / v with the causal flag; the math backend, whose batched bf16 products are not
         used here, is excluded, and where no fused kernel takes the shape the fp32 path runs.
@@ -453,6 +454,8 @@ class Qwen2Runner:
             return logits.clone()
         if (use_cache or pos0 > 0) and (self.cache_k is None or pos0 + T > self.max_len):
             raise RuntimeError("cache too small: alloc_cache(max_len) first")
+        if T == 0:
+            return self.embed.new_empty((0, s.vocab))
         D, G = s.head_dim, s.group
         qn, kn = s.heads * D, s.kv_heads * D
         x = self.embed.index_select(0, ids.to(self.dev)).contiguous()
@@ -469,15 +472,27 @@ class Qwen2Runner:
                 return k.w4_linear_packed_swiglu(a, *self.packed[li]["wgu"])
             return k.w4_linear_swiglu(a, *self.layers[li]["wgu"], G)
 
-        for li, L in enumerate(self.layers):
-            qkv = lin(h, li, "wqkv")
-            if L["bqkv"] is not None:
-                qkv += L["bqkv"]
+        cached = use_cache or pos0 > 0
+        in_kernel = self._prompt_attention_kernel_ok(T, pos0)
+        # one workspace for the pass: the layers' launches follow each other on one stream
+        work = (k.prompt_attention_workspace(T, s.heads, s.kv_heads, pos0, device=self.dev)
+                if in_kernel else None)
+
+        def attention(qkv, bias, li):
+            """Bias, RoPE, KV append and attention of the fused projection's output."""
+            caches = (self.cache_k[li], self.cache_v[li]) if cached else (None, None)
+            k.prompt_qkv(qkv, bias, self.inv_freq, s.heads, s.kv_heads, D, pos0, *caches)
             q, kk, v = qkv[:, :qn], qkv[:, qn:qn + kn], qkv[:, qn + kn:]
-            k.rope(q, kk, self.inv_freq, s.heads, s.kv_heads, D, pos0)
-            if use_cache or pos0 > 0:
-                self._store_kv(li, kk, v, pos0)
-            a = self._prompt_attention(q, kk, v, pos0, li)
+            if not in_kernel:
+                if cached and pos0 == 0:  # the rotated heads of this chunk are in the cache
+                    kk, v = (c[:, :T].transpose(0, 1).reshape(T, kn) for c in caches)
+                return self._prompt_attention(q, kk, v, pos0, li)
+            if not cached:
+                caches = (x.unflatten(1, (s.kv_heads, D)).transpose(0, 1) for x in (kk, v))
+            return k.prompt_attention(q, *caches, s.heads, pos0, work=work)
+
+        for li, L in enumerate(self.layers):
+            a = attention(lin(h, li, "wqkv"), L["bqkv"], li)
             h = k.rmsnorm(x, lin(a, li, "wo"), L["ln_post"], s.eps)
             act = gate_up_swiglu(h, li)
             # the down output joins the residual stream under the norm that follows this layer
