@@ -15,6 +15,7 @@
 
 #include "../../include/nanoserve_decode.h"
 #include "w4_common.h"
+#include "w4_kernels.h"
 
 namespace ns {
 namespace {
@@ -172,6 +173,21 @@ __global__ void __launch_bounds__(256)
     for (int e = 0; e < 8; ++e) a[e] = silu_mul(a[e], b[e]);
     st16(orr, 16u * (threadIdx.x + 256u * j), pack8(a));
   }
+}
+
+// The same on one tensor whose columns are gate and up values interleaved in blocks of 8 (v16
+// pairs of 16-byte vectors): a thread per pair.
+__global__ void __launch_bounds__(256)
+    swiglu_interleaved_kernel(const uint16_t* __restrict__ gu, uint16_t* __restrict__ out, size_t pairs) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= pairs) return;
+  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(gu) + 2 * i;
+  float a[8], b[8];
+  unpack8(src[0], a);
+  unpack8(src[1], b);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) a[e] = silu_mul(a[e], b[e]);
+  reinterpret_cast<u32x4_t*>(out)[i] = pack8(a);
 }
 
 // ------------------------------------------------------------------ decode: bias + RoPE + cache
@@ -797,6 +813,12 @@ int scratch_address(void** out) {
 }
 
 }  // namespace
+
+void launch_swiglu_interleaved(const uint16_t* gu, uint16_t* out, int M, int N, hipStream_t st) {
+  const size_t pairs = (size_t)M * N / 16;
+  hipLaunchKernelGGL(swiglu_interleaved_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, st,
+                     gu, out, pairs);
+}
 }  // namespace ns
 
 extern "C" {

@@ -1,11 +1,11 @@
 /*
- * prompt_ops.h -- entry points behind Qwen2Runner's prompt pass (libnanoserve_amd.so), called by
- * nanoserve_amd/ops.py. Conventions of include/nanoserve_decode.h: caller-allocated device
+ * internal_ops.h -- entry points of libnanoserve_amd.so that nanoserve_amd/ops.py calls and the
+ * public headers do not declare. Conventions of include/nanoserve_decode.h: caller-allocated device
  * memory, bf16 tensors as void*, asynchronous on `stream`, no allocation, capturable; 0 on
  * success, -2 for rejected arguments (checked before any HIP call), else the hipError_t.
  */
-#ifndef NANOSERVE_PROMPT_OPS_H
-#define NANOSERVE_PROMPT_OPS_H
+#ifndef NANOSERVE_INTERNAL_OPS_H
+#define NANOSERVE_INTERNAL_OPS_H
 
 #include <stddef.h>
 
@@ -47,8 +47,28 @@ int ns_prompt_attention(const void* q, long long q_stride, const void* k, const 
                         long long kv_stride, long long kv_head_stride, void* out, void* work,
                         size_t work_bytes, int T, int Hq, int Hk, int pos0, void* stream);
 
+/*
+ * ns_w4_linear for any M >= 1: above 8 rows the prefill GEMM on M rows as they are (ns_w4_linear takes
+ * multiples of 128, and the reference's wrapper pads to them, python/nanoserve/ops.py:88-91). The
+ * other conditions and return codes are ns_w4_linear's.
+ */
+int ns_w4_linear_rows(const void* X, const void* Wq, const void* S, void* Y, int M, int N, int K,
+                      int G, void* stream);
+
+/*
+ * ns_w4_linear_swiglu for any M >= 1: above 8 rows the GEMM with the SwiGLU epilogue on M rows as
+ * they are; M = 2..8 the decode GEMV with SwiGLU in its output where G == 128 and K % 256 == 0
+ * up to 20480, and elsewhere ns_w4_linear into `tmp` [M][N] bf16 followed by the activation
+ * (g and u rounded to bf16 first in either form). tmp: the workspace function's bytes, 16-byte
+ * aligned, or NULL where those are 0. M = 2..8 need Y 16-byte aligned. The other conditions and return
+ * codes are ns_w4_linear_swiglu's.
+ */
+size_t ns_w4_linear_swiglu_rows_workspace(int M, int N, int K, int G);
+int ns_w4_linear_swiglu_rows(const void* X, const void* Wq, const void* S, void* Y, void* tmp,
+                             size_t tmp_bytes, int M, int N, int K, int G, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
 
-#endif /* NANOSERVE_PROMPT_OPS_H */
+#endif /* NANOSERVE_INTERNAL_OPS_H */

@@ -7,6 +7,7 @@
 
 #include "../../include/nanoserve_decode.h"
 #include "../../include/nanoserve_w4.h"
+#include "internal_ops.h"
 #include "w4_common.h"
 #include "w4_kernels.h"
 
@@ -36,10 +37,10 @@ int ns_w4_quantize(const void* W, void* Wq, void* S, int N, int K, int G, void* 
 
 namespace {
 
-// ns_w4_linear and ns_w4_linear_ws: the same checks and dispatch; `ws` (may be null) is the
-// K-split GEMV's partials buffer.
+// ns_w4_linear, ns_w4_linear_ws and ns_w4_linear_rows: the same checks and dispatch; `ws` (may be
+// null) is the K-split GEMV's partials buffer, `any_m` admits GEMMs whose M is no multiple of 128.
 int w4_linear(const void* X, const void* Wq, const void* S, void* Y, int M, int N, int K, int G,
-              void* ws, size_t ws_bytes, void* stream) {
+              void* ws, size_t ws_bytes, void* stream, bool any_m = false) {
   if (M <= 0 || N <= 0 || K <= 0 || G <= 0) return -2;
   if (!X || !Wq || !S || !Y) return -2;
   if (!aligned(X, 16) || !aligned(Wq, 16) || !aligned(S, 2) || !aligned(Y, 2)) return -2;
@@ -54,7 +55,7 @@ int w4_linear(const void* X, const void* Wq, const void* S, void* Y, int M, int 
     if (!fmt_ok) return -2;
     const ns::GemvArgs a{x, wq, s, y, M, N, K, G};
     e = ns::launch_gemv(a, ns::gemv_plan(M, N, K, G), st, static_cast<float*>(ws), ws_bytes);
-  } else if (M % 128 == 0 && N % 128 == 0 && fmt_ok) {
+  } else if ((any_m || M % 128 == 0) && N % 128 == 0 && fmt_ok) {
     const ns::GemmArgs a{x, wq, s, y, M, N, K, G};
     e = ns::launch_gemm(a, ns::gemm_plan(M, N, K, G), st);
   } else {
@@ -84,18 +85,51 @@ int ns_w4_linear_ws(const void* X, const void* Wq, const void* S, void* Y, int M
   return w4_linear(X, Wq, S, Y, M, N, K, G, need > 0 ? work : nullptr, work_bytes, stream);
 }
 
+int ns_w4_linear_rows(const void* X, const void* Wq, const void* S, void* Y, int M, int N, int K,
+                      int G, void* stream) {
+  return w4_linear(X, Wq, S, Y, M, N, K, G, nullptr, 0, stream, true);
+}
+
 int ns_w4_linear_swiglu(const void* X, const void* Wq, const void* S, void* Y, int M, int N,
                         int K, int G, void* stream) {
+  if (M != 1 && M % 128) return -2;
+  return ns_w4_linear_swiglu_rows(X, Wq, S, Y, nullptr, 0, M, N, K, G, stream);
+}
+
+size_t ns_w4_linear_swiglu_rows_workspace(int M, int N, int K, int G) {
+  if (M < 2 || M > 8 || N <= 0 || K <= 0 || G <= 0 || K % 32 || G % 32 || K % G) return 0;
+  return ns::gemv_plan(M, N, K, G).m8 ? 0 : static_cast<size_t>(M) * N * 2;
+}
+
+int ns_w4_linear_swiglu_rows(const void* X, const void* Wq, const void* S, void* Y, void* tmp,
+                             size_t tmp_bytes, int M, int N, int K, int G, void* stream) {
   if (M <= 0 || N <= 0 || K <= 0 || G <= 0 || N % 16) return -2;
   if (!X || !Wq || !S || !Y) return -2;
   if (!aligned(X, 16) || !aligned(Wq, 16) || !aligned(S, 2) || !aligned(Y, 2)) return -2;
   if (M == 1) return ns_w4_gemv_decode(X, nullptr, nullptr, nullptr, 0.f, nullptr, Wq, S, Y, N, K,
                                        G, 1, stream);
-  if (M % 128 || N % 128 || K % 32 || G % 32 || K % G || !ns::gemm_v2_ok(M, N, K, G)) return -2;
-  const ns::GemmArgs a{static_cast<const uint16_t*>(X), static_cast<const uint32_t*>(Wq),
-                       static_cast<const uint16_t*>(S), static_cast<uint16_t*>(Y), M, N, K, G};
-  const hipError_t e = ns::launch_gemm_swiglu(a, ns::gemm_plan(M, N, K, G),
-                                              static_cast<hipStream_t>(stream));
+  if (K % 32 || G % 32 || K % G) return -2;
+  const auto st = static_cast<hipStream_t>(stream);
+  const auto x = static_cast<const uint16_t*>(X);
+  const auto wq = static_cast<const uint32_t*>(Wq);
+  const auto s = static_cast<const uint16_t*>(S);
+  const auto y = static_cast<uint16_t*>(Y);
+  hipError_t e;
+  if (M <= 8) {
+    if (!aligned(Y, 16)) return -2;
+    const size_t need = ns_w4_linear_swiglu_rows_workspace(M, N, K, G);
+    if (need == 0) {
+      e = ns::launch_gemv_m8_swiglu(ns::GemvArgs{x, wq, s, y, M, N, K, G}, st);
+    } else {
+      if (!tmp || tmp_bytes < need || !aligned(tmp, 16)) return -2;
+      const auto gu = static_cast<uint16_t*>(tmp);
+      e = ns::launch_gemv(ns::GemvArgs{x, wq, s, gu, M, N, K, G}, ns::gemv_plan(M, N, K, G), st);
+      if (e == hipSuccess) ns::launch_swiglu_interleaved(gu, y, M, N, st);
+    }
+  } else {
+    if (N % 128 || !ns::gemm_v2_ok(M, N, K, G)) return -2;
+    e = ns::launch_gemm_swiglu(ns::GemmArgs{x, wq, s, y, M, N, K, G}, ns::gemm_plan(M, N, K, G), st);
+  }
   if (e != hipSuccess) return static_cast<int>(e);
   return last_status();
 }

@@ -1,12 +1,12 @@
 // The prompt pass's attention step for gfx950: bias + RoPE + KV append in one launch, and causal
-// grouped-query attention on bf16 matrix cores (contracts in prompt_ops.h). The reference does
+// grouped-query attention on bf16 matrix cores (contracts in internal_ops.h). The reference does
 // both with PyTorch ops (python/nanoserve/qwen.py:119-133, 147-151).
 #include <math.h>
 #include <stdint.h>
 
 #include <algorithm>
 
-#include "prompt_ops.h"
+#include "internal_ops.h"
 #include "w4_common.h"
 #include "w4_kernels.h"
 

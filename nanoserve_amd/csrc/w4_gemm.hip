@@ -373,33 +373,49 @@ __device__ __forceinline__ void wait_vmcnt_c() {
   __builtin_amdgcn_s_waitcnt(imm);
 }
 
-// K-split handoff of the GEMMs: group g hands its accumulators (MI x NJ vectors of R floats) to
-// group 0 in round g through pb (this wave's slice of the free LDS ring, lane-major: word r * 64
-// + lane); group 0 adds them in group order. Every wave of the workgroup calls it (it holds
-// barriers).
-template <int KS, int MI, int NJ, typename V>
-__device__ __forceinline__ void k_group_handoff(V (&acc)[MI][NJ], float* pb, int ks, int lane) {
+// K-split handoff of the GEMMs: groups 1 .. KS-1 hand their accumulators (MI x NJ vectors of R
+// floats) to group 0 through the free LDS ring `lds` (FLOATS floats; group g's wave wv of NWN in
+// lane-major order: word r * 64 + lane of its slice), and group 0 adds them in group order. Where
+// the ring holds every group's accumulators at once they go in one round; otherwise one group per
+// round. Every wave of the workgroup calls it (it holds barriers).
+template <int KS, int NWN, int FLOATS, int MI, int NJ, typename V>
+__device__ __forceinline__ void k_group_handoff(V (&acc)[MI][NJ], float* lds, int wv, int ks, int lane) {
   constexpr int R = sizeof(V) / sizeof(float);
-#pragma unroll 1
-  for (int g = 1; g < KS; ++g) {
-    if (ks == g) {
+  constexpr int WAVE = kWave * MI * NJ * R;  // floats per wave
+  constexpr bool kOneRound = (KS - 1) * NWN * WAVE <= FLOATS;
+  float* pb = lds + wv * WAVE + lane;
+  auto put = [&](float* p) {
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+      for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int r = 0; r < R; ++r) pb[((i * NJ + j) * R + r) * kWave + lane] = acc[i][j][r];
-    }
-    lds_barrier();
+        for (int r = 0; r < R; ++r) p[((i * NJ + j) * R + r) * kWave] = acc[i][j][r];
+  };
+  auto add = [&](const float* p) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[i][j][r] += p[((i * NJ + j) * R + r) * kWave];
+  };
+  if constexpr (kOneRound) {
+    if (ks > 0) put(pb + (ks - 1) * NWN * WAVE);
+    lds_sync();
     if (ks == 0) {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-          for (int r = 0; r < R; ++r) acc[i][j][r] += pb[((i * NJ + j) * R + r) * kWave + lane];
+#pragma unroll 1
+      for (int g = 1; g < KS; ++g) add(pb + (g - 1) * NWN * WAVE);
     }
-    lds_barrier();
+    lds_sync();  // group 0's waves have read their slices before the epilogue reuses the LDS
+  } else {
+#pragma unroll 1
+    for (int g = 1; g < KS; ++g) {
+      if (ks == g) put(pb);
+      lds_sync();
+      if (ks == 0) add(pb);
+      lds_sync();
+    }
   }
 }
 
@@ -407,7 +423,7 @@ __device__ __forceinline__ void k_group_handoff(V (&acc)[MI][NJ], float* pb, int
 // split K inside the workgroup. Group ks computes 64-k blocks ks, ks + KS, ... into its own
 // accumulators through its own part of the LDS ring (step t loads and computes block t KS + ks
 // in every group); at the end groups 1 .. KS-1 hand their accumulators to group 0 through LDS,
-// one group per round, and group 0 adds them in group order and stores the tile.
+// and group 0 adds them in group order and stores the tile.
 // 256-row tiles carry 128 accumulators per lane: the launch bound asks for two waves per SIMD
 // (two four-wave workgroups per CU, or one eight-wave workgroup with KS = 2) so the compiler
 // keeps them in VGPRs beside the operands.
@@ -603,7 +619,7 @@ __global__ __launch_bounds__(NWN * KS * kWave, BM >= 256 && KS == 1 ? 2 : 1) voi
   wait_vmcnt_c<0>();  // the trailing out-of-range loads have landed before the LDS is reused
   lds_barrier();      // every wave is done reading the ring
   if constexpr (KS > 1) {
-    k_group_handoff<KS>(acc, reinterpret_cast<float*>(As) + wv * (kWave * MI * NJ * 16), ks, lane);
+    k_group_handoff<KS, NWN, sizeof(As) / 4>(acc, reinterpret_cast<float*>(As), wv, ks, lane);
     if (ks != 0) return;  // no barrier follows
   }
   if constexpr (SW)
@@ -742,8 +758,8 @@ __device__ __forceinline__ uint32_t dequant_pair_bf16_pk(uint32_t w, uint32_t vm
 //    WD steps ahead are issued at the step's first block into a register ring of WD + 1 slots.
 //  * KS > 1 (tile grids that do not fill the chip, e.g. the 7B down projection): KS groups of
 //    NWN waves split the tile columns (group g takes columns g, g + KS, ..., through its own
-//    two stages); groups 1 .. KS-1 then hand their accumulators to group 0 through LDS, one
-//    group per round, and group 0 adds them in group order.
+//    two stages); groups 1 .. KS-1 then hand their accumulators to group 0 through LDS, and
+//    group 0 adds them in group order.
 //  * Epilogue (group 0): each wave rounds its BM x 32 sub-tile to bf16 into a private part of
 //    the (then free) LDS ring and stores 16-byte row segments.
 template <int BM, int NWN, int KS, int WD, bool SW = false>
@@ -919,7 +935,7 @@ void w4_gemm_pk_kernel(const uint16_t* __restrict__ A, const uint32_t* __restric
   lds_barrier();  // every wave is done with the ring
 
   if constexpr (KS > 1) {
-    k_group_handoff<KS>(acc, reinterpret_cast<float*>(As) + wv * (kWave * MI * NJ * 4), ks, lane);
+    k_group_handoff<KS, NWN, sizeof(As) / 4>(acc, reinterpret_cast<float*>(As), wv, ks, lane);
     if (ks != 0) return;  // no barrier follows
   }
   if constexpr (SW)
@@ -945,6 +961,11 @@ constexpr TileCfg kCfgs[] = {
     {256, 128, 1.00f},  // 7: v2, BM 256, K split over 2 wave groups of 4, 2 stages, one per CU
     {128, 64, 1.00f},   // 8: v2, BM 128, K split over 4 wave groups of 2, 2 stages, one per CU
     {64, 64, 1.00f},    // 9: v2, BM 64, K split over 4 wave groups of 2, 2 stages, two per CU
+    {32, 32, 1.00f},    // 10: v2, BM 32, K split over 8 waves, 4 stages, one per CU
+    {32, 64, 1.00f},    // 11: v2, BM 32, K split over 4 wave groups of 2, 4 stages, two per CU
+    {64, 32, 1.00f},    // 12: v2, BM 64, K split over 4 waves, 4 stages, two per CU
+    {32, 64, 1.00f},    // 13: v2, BM 32, K split over 4 wave groups of 2, 3 stages, three per CU
+    {64, 128, 1.00f},   // 14: v2, BM 64, K split over 2 wave groups of 4, 4 stages, two per CU
 };
 
 }  // namespace
@@ -992,6 +1013,27 @@ GemmPlan gemm_plan(int M, int N, int K, int G) {
     if (tiles <= cus) {
       const long t128x64 = (long)((M + 127) / 128) * ((N + 63) / 64);
       c = tiles < cus && 4 * t128x64 >= 3 * cus && t128x64 <= cus ? 8 : 2 * tiles > cus ? 5 : 9;
+    }
+    // Few rows, or few tiles: the loop over K is a chain of load latencies, so smaller tiles (more
+    // of the chip, more K groups) with three blocks of activations in flight instead of one.
+    // us, the plan above in brackets:
+    //  * 32 x 32 tiles on eight K groups when they fit the CUs once: 4608 x 3584 at M = 16 9.6
+    //    [17.4], M = 32 10.8 [17.2]; 3584 x 18944 at M = 16 32.4 [70.9], M = 64 42.0 [71.2]; 1536 x
+    //    8960 at M = 100 18.1 [35.1].
+    //  * else 32 x 64 tiles on four groups, again at most one per CU: 4608 x 3584 at M = 64 13.4
+    //    [17.3], 3584 x 3584 at M = 100 12.5 [15.8], 3584 x 18944 at M = 128 56.0 [70.5].
+    //  * else 64 x 32 tiles on four groups likewise: 1536 x 8960 at M = 256 28.3 [33.9].
+    //  * wide layers, more tiles than CUs, M <= 32: 32 x 64 tiles with three stages, three per CU
+    //    (37888 x 3584 at M = 16 33.0 [51], 17920 x 1536 10.8 [16]); M <= 64: 64 x 128 tiles on two
+    //    groups (17920 x 1536 at M = 64 12.8 [16.6], 37888 x 3584 44.0 [51.9]).
+    // Past these the plans above are level or ahead (4608 x 3584 at M = 128 17.1 against 18.0).
+    auto count = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    if (c == 9 || M <= 64) {
+      if (count(32, 32) <= cus) c = 10;
+      else if (count(32, 64) <= cus) c = 11;
+      else if (count(64, 32) <= cus) c = 12;
+      else if (M <= 32) c = 13;
+      else if (M <= 64) c = 14;
     }
     return GemmPlan{c, kCfgs[c].bm, kCfgs[c].bn};
   }
@@ -1121,6 +1163,26 @@ hipError_t launch_gemm(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
       hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 2, 2, false, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
                          a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
       return hipSuccess;
+    case 10:
+      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 1, 4, false, 8>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 11:
+      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 4, false, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 12:
+      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 1, 4, false, 4>), grid, dim3(256), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 13:
+      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 3, false, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 14:
+      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 4, false, 2>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
     default:
       return hipErrorInvalidValue;
   }
@@ -1152,6 +1214,26 @@ hipError_t launch_gemm_swiglu(const GemmArgs& a, const GemmPlan& p, hipStream_t 
     case 9:
       hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 2, 2, true, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
                          a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 10:
+      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 1, 4, true, 8>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 11:
+      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 4, true, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 12:
+      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 1, 4, true, 4>), grid, dim3(256), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 13:
+      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 3, true, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 14:
+      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 4, true, 2>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
+                         a.M, a.N, a.K, ilog2(a.G));
       return hipSuccess;
     default:
       return hipErrorInvalidValue;

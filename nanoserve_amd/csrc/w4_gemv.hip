@@ -1059,7 +1059,10 @@ __device__ __forceinline__ void xpose_rows(u32x4_t (&r)[4]) {
 //    wave leaves its per-tile partials (4 rows m x 1 row n per useful lane) in a double-
 //    buffered LDS table; after the group's barrier GT waves sum them over waves and halves
 //    and store Y.
-template <int CW, int GT, int R>
+//  * SW: the rows are gate and up rows interleaved in blocks of 8, so tiles 2 i and 2 i + 1 of a
+//    group are the gate and up rows of the same eight features: the wave that sums one sums both
+//    and stores bf16(silu(g) * u) of the two rounded values to Y [M][N / 2] (ks = 1).
+template <int CW, int GT, int R, bool SW = false>
 __global__ __launch_bounds__(1024) void w4_gemv_m8_kernel(
     const uint16_t* __restrict__ X, const uint32_t* __restrict__ Wq,
     const uint16_t* __restrict__ S, uint16_t* __restrict__ Y, int M, int N, int K, int ks,
@@ -1219,18 +1222,26 @@ __global__ __launch_bounds__(1024) void w4_gemv_m8_kernel(
     // output (m = lane / 8, row nl = lane % 8) of tile u: half h of every wave sits at slot
     // (8 h + nl) * 2 + m / 4 (compact table) or lane (j = nl + 8 h, kq = 2 h + m / 4), register
     // m % 4
-    for (int u = (wv - it % NW + NW) % NW; u < GT; u += NW) {  // every tile, also when NW < GT
-      const int om = lane >> 3, on = lane & 7;
-      const int q0 = kCompact ? 4 * (2 * on + (om >> 2)) + (om & 3)
-                              : 4 * (on + 16 * (om >> 2)) + (om & 3);
-      const int q1 = kCompact ? q0 + 4 * 16 : q0 + 4 * (8 + 32);
+    const int om = lane >> 3, on = lane & 7;
+    const int q0 = kCompact ? 4 * (2 * on + (om >> 2)) + (om & 3)
+                            : 4 * (on + 16 * (om >> 2)) + (om & 3);
+    const int q1 = kCompact ? q0 + 4 * 16 : q0 + 4 * (8 + 32);
+    auto tile_sum = [&](int u) {
       float v = 0.f;
       for (int w = 0; w < NW; ++w) {
         const float* pw = reinterpret_cast<const float*>(rb + (w * GT + u) * kSlots);
         v += pw[q0] + pw[q1];
       }
+      return v;
+    };
+    constexpr int US = SW ? 2 : 1;  // tiles per output block
+    for (int u = US * ((wv - it % NW + NW) % NW); u < GT; u += US * NW) {  // every tile, also when NW < GT
+      const float v = tile_sum(u);
       const int n = 8 * (GT * g + u) + on;
-      if (om < M && n < N) {
+      if constexpr (SW) {
+        const float y = silu_mul(round_bf16(v), round_bf16(tile_sum(u + 1)));
+        if (om < M && n < N) Y[(size_t)om * (N >> 1) + 4 * (GT * g + u) + on] = (uint16_t)f32_to_bf16_rne(y);
+      } else if (om < M && n < N) {
         if (ks == 1)
           Y[(size_t)om * N + n] = (uint16_t)f32_to_bf16_rne(v);
         else
@@ -1573,9 +1584,9 @@ hipError_t launch_m1(const GemvArgs& a, hipStream_t st, const M1Fuse& fz = M1Fus
 }
 
 // Workgroups per CU the M = 2..8 kernel can hold (occupancy), or a negative error.
-template <int CW, int GT, int R>
+template <int CW, int GT, int R, bool SW = false>
 int m8_per_cu(int nw, hipError_t* err) {
-  const void* fn = reinterpret_cast<const void*>(&w4_gemv_m8_kernel<CW, GT, R>);
+  const void* fn = reinterpret_cast<const void*>(&w4_gemv_m8_kernel<CW, GT, R, SW>);
   const hipError_t attr = cached_max_dynamic_lds(fn, 160 * 1024);
   *err = attr;
   if (attr != hipSuccess) return 0;
@@ -1596,10 +1607,10 @@ struct M8Split {
   float* part = nullptr;
 };
 
-template <int CW, int GT, int R>
+template <int CW, int GT, int R, bool SW = false>
 hipError_t launch_m8(const GemvArgs& a, int nw, int cap, const M8Split& sp, hipStream_t st) {
   hipError_t e;
-  const int per_cu = m8_per_cu<CW, GT, R>(nw, &e);
+  const int per_cu = m8_per_cu<CW, GT, R, SW>(nw, &e);
   if (e != hipSuccess) return e;
   const size_t lds = m8_bytes(nw, CW, GT);
   int cus = 0;
@@ -1608,7 +1619,7 @@ hipError_t launch_m8(const GemvArgs& a, int nw, int cap, const M8Split& sp, hipS
   const int ngroups = ((a.N + 7) / 8 + GT - 1) / GT;
   // workgroups per slice: every slice serves every group, so the grid is a multiple of ks
   const int per_slice = max(1, min(ngroups, min(max(per_cu, 1), cap) * cus / sp.ks));
-  hipLaunchKernelGGL((w4_gemv_m8_kernel<CW, GT, R>), dim3(per_slice * sp.ks), dim3(nw * kWave), lds,
+  hipLaunchKernelGGL((w4_gemv_m8_kernel<CW, GT, R, SW>), dim3(per_slice * sp.ks), dim3(nw * kWave), lds,
                      st, a.X, a.Wq, a.S, a.Y, a.M, a.N, a.K, sp.ks, sp.part);
   if (sp.ks > 1) {
     const int mn = a.M * a.N;
@@ -1641,14 +1652,14 @@ hipError_t launch_m8c(const GemvArgs& a, hipStream_t st) {
 // M = 8 this picks 16-row groups at one workgroup per CU for qkv (4608 x 3584: 256 workgroups
 // against 144 with 32-row groups, 6.89 -> 6.63 us) and o (3584 x 3584), and 32-row groups for
 // gate/up (37888 x 3584, one workgroup per CU), each the fastest of the candidates measured.
-template <int CW>
+template <int CW, bool SW = false>
 hipError_t launch_m8_auto(const GemvArgs& a, int nw, const M8Split& sp, hipStream_t st) {
   int cus = 0;
   hipError_t e = cached_cu_count(&cus);
   if (e != hipSuccess) return e;
-  const int pc2 = m8_per_cu<CW, 2, 2>(nw, &e);
+  const int pc2 = m8_per_cu<CW, 2, 2, SW>(nw, &e);
   if (e != hipSuccess) return e;
-  const int pc4 = m8_per_cu<CW, 4, 4>(nw, &e);
+  const int pc4 = m8_per_cu<CW, 4, 4, SW>(nw, &e);
   if (e != hipSuccess) return e;
   const double xb = 2.0 * a.M * a.K / sp.ks, rowb = 0.5 * a.K / sp.ks;
   const int ntiles = (a.N + 7) / 8;
@@ -1657,7 +1668,7 @@ hipError_t launch_m8_auto(const GemvArgs& a, int nw, const M8Split& sp, hipStrea
   // barriers: 28672 x 4096 17.8 / 17.2 -> 16.6 / 16.0; the 7B gate/up already took them); with
   // six waves or fewer, two workgroups per CU at least (17920 x 1536 8.3 / 8.0 -> 6.5 / 6.1).
   if (CW == 1 && sp.ks == 1 && nw >= 12 && (ntiles + 3) / 4 >= cus && pc4 >= 1)
-    return launch_m8<CW, 4, 4>(a, nw, 1, sp, st);
+    return launch_m8<CW, 4, 4, SW>(a, nw, 1, sp, st);
   const int min_cap = sp.ks == 1 && nw <= 6 ? 2 : 1;
   struct Cand {
     int gt, cap, wgs;
@@ -1682,8 +1693,8 @@ hipError_t launch_m8_auto(const GemvArgs& a, int nw, const M8Split& sp, hipStrea
       bcap = cand[i].cap;
       bwgs = cand[i].wgs;
     }
-  if (bgt == 4) return launch_m8<CW, 4, 4>(a, nw, bcap, sp, st);
-  return launch_m8<CW, 2, 2>(a, nw, bcap, sp, st);
+  if (bgt == 4) return launch_m8<CW, 4, 4, SW>(a, nw, bcap, sp, st);
+  return launch_m8<CW, 2, 2, SW>(a, nw, bcap, sp, st);
 }
 
 template <int MP, int NW, int CW, int ST, int DPW>
@@ -1966,6 +1977,25 @@ namespace {
 
 // The norm prologue keeps its vectors live across the row reduction, so it is compiled for
 // as few vectors per thread as the row needs (registers decide how many workgroups fit a CU).
+}  // namespace
+
+// The M = 2..8 GEMV with SwiGLU in its output; only plans with p.m8, in one pass over K.
+hipError_t launch_gemv_m8_swiglu(const GemvArgs& a, hipStream_t st) {
+  int cw = 0, nw = 0;
+  const M8Split sp;
+  m8_shape(a.K, 1, &cw, &nw);
+  switch (cw) {
+    case 1: return launch_m8_auto<1, true>(a, nw, sp, st);
+    case 2: return launch_m8_auto<2, true>(a, nw, sp, st);
+    case 3: return launch_m8<3, 2, 2, true>(a, nw, 2, sp, st);
+    case 4: return launch_m8<4, 2, 2, true>(a, nw, 2, sp, st);
+    case 5: return launch_m8<5, 2, 2, true>(a, nw, 2, sp, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+namespace {
+
 template <int NW, int GR, int YM, int XV>
 hipError_t launch_m1_norm(const GemvArgs& a, const M1Fuse& fz, hipStream_t st, int wpc) {
   if (fz.radd) return launch_m1<NW, 2, GR, kXNormAdd, YM, XV>(a, st, fz, wpc);

@@ -81,6 +81,12 @@ hipError_t launch_gemv_attn(const GemvArgs& a, const GemvPlan& p, const M1Fuse& 
 hipError_t launch_gemv_fused(const GemvArgs& a, const GemvPlan& p, const M1Fuse& fz, bool norm,
                              bool swiglu, hipStream_t st, int* reject);
 
+// The M = 2..8 GEMV (plans with p.m8) with SwiGLU in its output: rows interleaved gate/up in blocks
+// of 8, Y [M][N/2].
+hipError_t launch_gemv_m8_swiglu(const GemvArgs& a, hipStream_t st);
+// out [M][N/2] = bf16(silu(g) * u) of gu [M][N] with columns interleaved in blocks of 8.
+void launch_swiglu_interleaved(const uint16_t* gu, uint16_t* out, int M, int N, hipStream_t st);
+
 struct GemmArgs {
   const uint16_t* A;   // X [M][K] bf16
   const uint32_t* Wq;  // [N][K/8]

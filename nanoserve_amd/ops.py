@@ -50,10 +50,14 @@ SIGNATURES["ns_probe_read"] = [_VP, _SZ, _VP, _I32, _I32, _I32, _VP]
 SIGNATURES["ns_probe_empty"] = [_I32, _I32, _VP]
 SIGNATURES["ns_probe_linear_loop"] = [_VP] * 7 + [_I32, _I32, _VP]
 RESTYPES = {"ns_decode_attention_workspace": _SZ, "ns_w4_gptq_workspace": _SZ,
-            "ns_w4_linear_workspace": _SZ, "ns_prompt_attention_workspace": _SZ}
-# Entry points of this package's own callers (csrc/prompt_ops.h), not part of the public ABI.
+            "ns_w4_linear_workspace": _SZ, "ns_prompt_attention_workspace": _SZ,
+            "ns_w4_linear_swiglu_rows_workspace": _SZ}
+# Entry points of this package's own callers (csrc/internal_ops.h), not part of the public ABI.
 INTERNAL_SIGNATURES = {
     "ns_prompt_qkv": [_VP] * 5 + [_I32] * 6 + [_VP],
+    "ns_w4_linear_rows": [_VP] * 4 + [_I32] * 4 + [_VP],
+    "ns_w4_linear_swiglu_rows_workspace": [_I32] * 4,
+    "ns_w4_linear_swiglu_rows": [_VP] * 5 + [_SZ] + [_I32] * 4 + [_VP],
     "ns_prompt_attention_workspace": [_I32] * 4,
     "ns_prompt_attention": [_VP, _I64, _VP, _VP, _I64, _I64, _VP, _VP, _SZ, _I32, _I32, _I32, _I32,
                             _VP],
@@ -88,6 +92,12 @@ def _check_out(out: torch.Tensor, like: torch.Tensor) -> torch.Tensor:
     if out.shape != like.shape or not out.is_contiguous():
         raise ValueError(f"out must be a contiguous tensor of shape {tuple(like.shape)}")
     return out
+
+
+def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
+    """A contiguous tensor at a 16-byte aligned address: x, or a copy of a view that starts at
+    another one."""
+    return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
 class Kernels:
@@ -131,9 +141,8 @@ class Kernels:
 
     def w4_linear_swiglu(self, x, Wq, S, group=128, out=None):
         """x [M, K] bf16 -> [M, N // 2] bf16 = swiglu of x @ deq(Wq, S)^T whose rows are gate and
-        up rows interleaved in blocks of 8 (``qwen.interleave_gate_up``): one launch for M = 1
-        and M % 128 == 0 (ns_w4_linear_swiglu). Other M pad with zero rows to a multiple of 128
-        above 8, and run as ``w4_linear`` + ``swiglu`` for M = 2..8 (not in the reference,
+        up rows interleaved in blocks of 8 (``qwen.interleave_gate_up``): one launch, except for
+        the M = 2..8 shapes whose GEMV has no SwiGLU output, which take two (not in the reference,
         whose MLP is swiglu(linear(h, "g"), linear(h, "u")), qwen.py:159)."""
         _require_gpu_tensor(x, "x", torch.bfloat16)
         _require_gpu_tensor(Wq, "Wq", torch.int32)
@@ -149,24 +158,16 @@ class Kernels:
                 raise ValueError(f"out must be a contiguous tensor of shape {(M, I)}")
         if M == 0:
             return out if out is not None else x.new_empty((0, I))
-        if 2 <= M <= 8:
-            gu = self.w4_linear(x, Wq, S, group).view(M, I // 8, 2, 8)
-            return self.swiglu(gu[:, :, 0].reshape(M, I), gu[:, :, 1].reshape(M, I), out=out)
-        Mp = M if M == 1 else ((M + 127) // 128) * 128
-        if Mp != M:
-            x = torch.cat([x, x.new_zeros(Mp - M, K)])
         x = x.contiguous()
-        y = out if out is not None and Mp == M else torch.empty((Mp, I), dtype=torch.bfloat16,
-                                                                 device=x.device)
-        rc = self.lib.ns_w4_linear_swiglu(x.data_ptr(), Wq.contiguous().data_ptr(),
-                                          S.contiguous().data_ptr(), y.data_ptr(), Mp, N, K,
-                                          group, self._stream())
+        if M > 8 and M % 128:
+            x = _aligned_rows(x)
+        n = int(self.lib.ns_w4_linear_swiglu_rows_workspace(M, N, K, group))
+        y = torch.empty((M, I), dtype=torch.bfloat16, device=x.device) if out is None else out
+        tmp = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
+        rc = self.lib.ns_w4_linear_swiglu_rows(
+            x.data_ptr(), Wq.contiguous().data_ptr(), S.contiguous().data_ptr(), y.data_ptr(),
+            None if tmp is None else tmp.data_ptr(), n, M, N, K, group, self._stream())
         self._check(rc, "ns_w4_linear_swiglu")
-        if Mp != M:
-            y = y[:M]
-            if out is not None:
-                out.copy_(y)
-                return out
         return y
 
     def w4_gptq(self, W, U, group=128):
@@ -201,10 +202,9 @@ class Kernels:
     def w4_linear(self, x, Wq, S, group=128, out=None, work=None):
         """x [M, K] bf16 -> y [M, N] bf16 = x @ deq(Wq, S)^T. Reference ops.py:85-97.
 
-        M <= 8 runs natively (the reference pads 3 -> 4 and 5..7 -> 8 with zero rows, which
-        does not change any output row); larger M is padded with zero rows up to a multiple
-        of 128, as the reference does. ``out`` (not in the reference): a contiguous [M, N]
-        bf16 tensor to write instead of a new one, for M that needs no padding. ``work`` (not in
+        Any M runs natively (the reference pads 3 -> 4 and 5..7 -> 8 with zero rows, and larger M
+        up to a multiple of 128, which does not change any output row). ``out`` (not in the reference): a contiguous [M, N]
+        bf16 tensor to write instead of a new one, for M <= 8 and multiples of 128 (the M the reference does not pad). ``work`` (not in
         the reference): a workspace from ``w4_linear_workspace``; with it the M = 2..8 GEMV
         may split long rows over K (ns_w4_linear_ws), without it no shape is split
         (ns_w4_linear)."""
@@ -213,33 +213,34 @@ class Kernels:
         _require_gpu_tensor(S, "S", torch.bfloat16)
         M, K = x.shape
         N = Wq.shape[0]
-        Mp = M if M <= 8 else ((M + 127) // 128) * 128
+        padded = M > 8 and M % 128 != 0  # in the reference: ``out`` does not apply there
         if M == 0:
-            Mp = 1
-        if Mp != M:
-            x = torch.cat([x, x.new_zeros(Mp - M, K)])
+            x = x.new_zeros(1, K)
         x = x.contiguous()
+        if padded:
+            x = _aligned_rows(x)
         Wq = Wq.contiguous()
         S = S.contiguous()
         if out is not None:
             _require_gpu_tensor(out, "out", torch.bfloat16)
-            if Mp != M or tuple(out.shape) != (M, N) or not out.is_contiguous():
+            if M == 0 or padded or tuple(out.shape) != (M, N) or not out.is_contiguous():
                 raise ValueError(f"out must be a contiguous [{M}, {N}] tensor and M must need "
                                  "no padding")
             y = out
         else:
-            y = torch.empty((Mp, N), dtype=torch.bfloat16, device=x.device)
-        if work is None:
-            rc = self.lib.ns_w4_linear(x.data_ptr(), Wq.data_ptr(), S.data_ptr(), y.data_ptr(), Mp,
-                                       N, K, group, self._stream())
+            y = torch.empty((max(M, 1), N), dtype=torch.bfloat16, device=x.device)
+        if work is not None:
+            _require_gpu_tensor(work, "work", torch.uint8)
+        if work is None or padded:
+            rc = self.lib.ns_w4_linear_rows(x.data_ptr(), Wq.data_ptr(), S.data_ptr(), y.data_ptr(),
+                                            max(M, 1), N, K, group, self._stream())
             self._check(rc, "ns_w4_linear")
         else:
-            _require_gpu_tensor(work, "work", torch.uint8)
             rc = self.lib.ns_w4_linear_ws(x.data_ptr(), Wq.data_ptr(), S.data_ptr(), y.data_ptr(),
-                                          Mp, N, K, group, work.data_ptr(), work.numel(),
+                                          max(M, 1), N, K, group, work.data_ptr(), work.numel(),
                                           self._stream())
             self._check(rc, "ns_w4_linear_ws")
-        return y if Mp == M else y[:M]
+        return y if M else y[:0]
 
     # ------------------------------------------------------------------ decoder-step operators
     def rmsnorm(self, x, r, w, eps, out=None):
@@ -485,7 +486,7 @@ class Kernels:
                    v_cache=None):
         """T prompt tokens at positions pos0 ..: bias add + RoPE of the fused projection output
         qkv [T, (Hq + 2Hk) * D], q heads in place, k and v heads into rows pos0 .. of one layer's
-        k_cache / v_cache [Hk, max_len, D], or in place without them (csrc/prompt_ops.h). The
+        k_cache / v_cache [Hk, max_len, D], or in place without them (csrc/internal_ops.h). The
         reference does this with PyTorch ops and ns_rope (qwen.py:119-122, 147-151)."""
         _require_gpu_tensor(qkv, "qkv", torch.bfloat16)
         _require_gpu_tensor(inv_freq, "inv_freq", torch.float32)
