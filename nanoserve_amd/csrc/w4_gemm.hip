@@ -853,21 +853,34 @@ void w4_gemm_pk_kernel(const uint16_t* __restrict__ A, const uint32_t* __restric
       sc[jj] = bf16_bits_to_f32(r.s[jj] & 0xffffu);
       nb[jj] = -1032.f * sc[jj];
     }
-    u32x4_t b0[NJ], b1[NJ];
+    // A fragments f = MI s2 + i: chunk 4 s2 + kg of rows 16 i + fr. Three are in flight (an LDS read
+    // takes longer than the two MFMAs of one fragment; with one in flight, us: 3584 x 18944 at
+    // M = 700 153.8 -> 146.1, 4608 x 3584 at M = 512 33.2 -> 31.0, 37888 x 3584 at M = 2048 488 -> 485;
+    // four spill at 128 registers).
+    constexpr int AD = 3;
+    u32x4_t af[AD], b0[NJ], b1[NJ];
+    auto a_read = [&](int f) {
+      const int row = 16 * (f % MI) + fr;
+      const int ch = (4 * (f / MI) + kg) ^ ((row >> 1) & 7);
+      af[f % AD] = *reinterpret_cast<const u32x4_t*>(&as[row * BK + 8 * ch]);
+    };
+#pragma unroll
+    for (int f = 0; f < AD; ++f) a_read(f);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int jj = 0; jj < NJ; ++jj) b0[jj] = dequant_word_bf16_pk(r.w[jj][2 * H], vmask, sc[jj], nb[jj]);
     constexpr int PER = (4 * NJ + MI - 1) / MI;  // second-step pairs per row block
 #pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int row = 16 * i + fr;
-      const int ch = kg ^ ((row >> 1) & 7);
-      const u32x4_t af = *reinterpret_cast<const u32x4_t*>(&as[row * BK + 8 * ch]);
+    for (int f = 0; f < 2 * MI; ++f) {
+      const int i = f % MI;
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj)
-        acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(af), as_bf16x8(b0[jj]), acc[i][jj], 0, 0, 0);
+        acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            as_bf16x8(af[f % AD]), as_bf16x8(f < MI ? b0[jj] : b1[jj]), acc[i][jj], 0, 0, 0);
+      if (f + AD < 2 * MI) a_read(f + AD);
 #pragma unroll
       for (int p = 0; p < PER; ++p) {
-        const int q = PER * i + p;  // pair q % 4 of word q / 4
+        const int q = PER * f + p;  // pair q % 4 of word q / 4
         if (q < 4 * NJ) {
           const int jj = q >> 2;
           const uint32_t wd = r.w[jj][2 * H + 1];
@@ -881,16 +894,7 @@ void w4_gemm_pk_kernel(const uint16_t* __restrict__ A, const uint32_t* __restric
           b1[jj][q & 3] = v;
         }
       }
-      __builtin_amdgcn_sched_barrier(0x0100);  // only LDS reads may move across
-    }
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int row = 16 * i + fr;
-      const int ch = (4 + kg) ^ ((row >> 1) & 7);
-      const u32x4_t af = *reinterpret_cast<const u32x4_t*>(&as[row * BK + 8 * ch]);
-#pragma unroll
-      for (int jj = 0; jj < NJ; ++jj)
-        acc[i][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(af), as_bf16x8(b1[jj]), acc[i][jj], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -966,6 +970,11 @@ constexpr TileCfg kCfgs[] = {
     {64, 32, 1.00f},    // 12: v2, BM 64, K split over 4 waves, 4 stages, two per CU
     {32, 64, 1.00f},    // 13: v2, BM 32, K split over 4 wave groups of 2, 3 stages, three per CU
     {64, 128, 1.00f},   // 14: v2, BM 64, K split over 2 wave groups of 4, 4 stages, two per CU
+    {96, 64, 1.00f},    // 15: v2, BM 96, K split over 4 wave groups of 2, 2 stages, one per CU
+    {64, 128, 1.00f},   // 16: v2, BM 64, K split over 2 wave groups of 4, 2 stages
+    {96, 128, 1.00f},   // 17: v2, BM 96, K split over 2 wave groups of 4, 2 stages
+    {160, 128, 1.00f},  // 18: v2, BM 160, K split over 2 wave groups of 4, 2 stages
+    {192, 128, 1.00f},  // 19: v2, BM 192, K split over 2 wave groups of 4, 2 stages
 };
 
 }  // namespace
@@ -983,57 +992,39 @@ GemmPlan gemm_plan(int M, int N, int K, int G) {
   int cus = 256;  // the device's CU count (a failed query leaves MI355X's; the launch reports it)
   if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;
   if (gemm_v2_ok(M, N, K, G)) {
-    // Tile plans, measured on MI355X (A/B runs of the four config-4 shapes and the other shapes
-    // quoted):
-    //  * 128 x 128 tiles, three workgroups per CU: the default.
+    // Tile plans, measured on MI355X.
+    //  * A grid that fits the CUs once is bound by the time of one tile (its chain of loads over K,
+    //    then the arithmetic of its CU): the plan with the smallest tiles that still fits, K split
+    //    over as many wave groups as its LDS ring allows, with three blocks of activations in
+    //    flight for the smallest. Times of one round at K = 3584 / 18944, us: 32 x 32 9.9 / 42, 32 x
+    //    64 12.5 / 50, 64 x 32 13.7 / 54, 64 x 64 15.6 / 68, 96 x 64 19.5 / 82, 64 x 128 22 / 108,
+    //    128 x 64 23 / 100, 96 x 128 29 / 134, 128 x 128 33 / 155, 160 x 128 38 / 185, 192 x 128 45 /
+    //    215; 64 x 128 and 128 x 64 change places at K = 8192 (two K groups against four).
+    //    Against the 64 x 64, 128 x 64 and 128 x 128 plans alone: 4608 x 3584 at M = 16 17.4 -> 9.6,
+    //    M = 64 17.3 -> 13.4, M = 600 32.9 -> 29.6, M = 1000 49.4 -> 41.2; 3584 x 18944 at M = 64 71.2 ->
+    //    42.0, M = 700 159 -> 137, M = 1200 237 -> 192; 1536 x 8960 at M = 100 35.1 -> 18.1, M = 700
+    //    52.2 -> 42.2. (192 x 128 against two rounds of 128 x 128: 3584 x 3584 at M = 1500 47.3
+    //    against 52.4.)
+    //  * More tiles than CUs, few rows: 32 x 64 tiles with three stages, three per CU, for M <= 32
+    //    (37888 x 3584 at M = 16 33.0 against 51 for 128 x 128, 17920 x 1536 10.8 against 16); 64 x
+    //    128 tiles with four stages for M <= 64 (17920 x 1536 12.8 against 16.6, 37888 x 3584 44.0
+    //    against 51.9).
+    //  * 256 x 128 tiles with K split over two groups of four waves, one eight-wave workgroup per
+    //    CU, when those tiles fill three quarters to all of the CUs once and K >= 8192: 3584 x 18944
+    //    at M = 2048 320 -> 301 and 303.6 -> 289.7 us on two boxes, 4096 x 14336 263 -> 244; with
+    //    short K (3584 x 3584: 68 -> 72) 128 x 128 stays.
     //  * 256 x 128 tiles (each wave 256 x 32: one dequantized weight word feeds eight MFMAs, not
     //    four), two workgroups per CU, when there are at least four rounds of them: gate/up at
     //    M = 2048 590 -> 555 us; with fewer rounds (gate/up M = 512) 128 x 128 is faster.
-    //  * 256 x 128 tiles with K split over two groups of four waves, one eight-wave workgroup per
-    //    CU (two waves per SIMD on one tile, the K loop halved), when those tiles fill three
-    //    quarters to all of the CUs once and K >= 8192: down 3584 x 18944 at M = 2048 320 -> 301
-    //    and 303.6 -> 289.7 us on two boxes, 4096 x 14336 263 -> 244 us; with short K (3584 x
-    //    3584: 68 -> 72) or 128 such tiles (half the CUs: 159 -> 206) 128 x 128 stays.
-    //  * When 128 x 128 tiles fill at most one round of the CUs, K split inside the workgroup:
-    //    128 x 64 tiles over four wave groups of two (each wave a 32-column slice), one eight-wave
-    //    workgroup per CU, when they fill three quarters to all of the CUs (down at M = 512:
-    //    121.8 -> 102.2 us, 4096 x 14336 at M = 512 98.8 -> 86.2); else, with more than half the
-    //    CUs holding a 128 x 128 tile, those tiles over two groups of four waves, two eight-wave
-    //    workgroups per CU (against the 64 x 64 plan below, us: 3584 x 18944 at M = 1024 219.1 ->
-    //    161.5, M = 768 210.3 -> 148.6, 3328 x 11008 at M = 1024 132.4 -> 93.9, qkv 4608 x 3584 at
-    //    M = 512 37.0 -> 32.6, 3584 x 3584 at M = 768 39.2 -> 32.7; at exactly one round, 4096 x
-    //    14336 at M = 1024, 144.5 -> 135.2 against 128 x 128 unsplit; where the 128 x 64 plan
-    //    applies it stays ahead: down at M = 512 95.3 against 146.4); else 64 x 64 tiles over
-    //    four groups of two, two per CU (down at M = 256 113.6 -> 65.2 us, 3584 x 3584 24.7 ->
-    //    17.8).
-    const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
-    const long tiles256 = (long)((M + 255) / 256) * ((N + 127) / 128);
-    const bool ks256 = tiles256 <= cus && 4 * tiles256 >= 3 * cus && K >= 8192;
-    int c = ks256 ? 7 : tiles256 >= 4 * cus ? 6 : 4;
-    if (tiles <= cus) {
-      const long t128x64 = (long)((M + 127) / 128) * ((N + 63) / 64);
-      c = tiles < cus && 4 * t128x64 >= 3 * cus && t128x64 <= cus ? 8 : 2 * tiles > cus ? 5 : 9;
-    }
-    // Few rows, or few tiles: the loop over K is a chain of load latencies, so smaller tiles (more
-    // of the chip, more K groups) with three blocks of activations in flight instead of one.
-    // us, the plan above in brackets:
-    //  * 32 x 32 tiles on eight K groups when they fit the CUs once: 4608 x 3584 at M = 16 9.6
-    //    [17.4], M = 32 10.8 [17.2]; 3584 x 18944 at M = 16 32.4 [70.9], M = 64 42.0 [71.2]; 1536 x
-    //    8960 at M = 100 18.1 [35.1].
-    //  * else 32 x 64 tiles on four groups, again at most one per CU: 4608 x 3584 at M = 64 13.4
-    //    [17.3], 3584 x 3584 at M = 100 12.5 [15.8], 3584 x 18944 at M = 128 56.0 [70.5].
-    //  * else 64 x 32 tiles on four groups likewise: 1536 x 8960 at M = 256 28.3 [33.9].
-    //  * wide layers, more tiles than CUs, M <= 32: 32 x 64 tiles with three stages, three per CU
-    //    (37888 x 3584 at M = 16 33.0 [51], 17920 x 1536 10.8 [16]); M <= 64: 64 x 128 tiles on two
-    //    groups (17920 x 1536 at M = 64 12.8 [16.6], 37888 x 3584 44.0 [51.9]).
-    // Past these the plans above are level or ahead (4608 x 3584 at M = 128 17.1 against 18.0).
-    auto count = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    if (c == 9 || M <= 64) {
-      if (count(32, 32) <= cus) c = 10;
-      else if (count(32, 64) <= cus) c = 11;
-      else if (count(64, 32) <= cus) c = 12;
-      else if (M <= 32) c = 13;
-      else if (M <= 64) c = 14;
+    //  * 128 x 128 tiles, three workgroups per CU: the rest.
+    auto count = [&](int c) { return (long)((M + kCfgs[c].bm - 1) / kCfgs[c].bm) * ((N + kCfgs[c].bn - 1) / kCfgs[c].bn); };
+    const int first = K >= 8192 ? 8 : 16, second = K >= 8192 ? 16 : 8;
+    int c = 0;
+    for (const int p : {10, 11, 12, 9, 15, first, second, 17, 5, 18, 19})
+      if (c == 0 && count(p) <= cus && (M > 64 || kCfgs[p].bm <= (M <= 32 ? 32 : 64))) c = p;
+    if (c == 0) {
+      const bool ks256 = count(7) <= cus && 4 * count(7) >= 3 * cus && K >= 8192;
+      c = M <= 32 ? 13 : M <= 64 ? 14 : ks256 ? 7 : count(6) >= 4l * cus ? 6 : 4;
     }
     return GemmPlan{c, kCfgs[c].bm, kCfgs[c].bn};
   }
@@ -1059,62 +1050,76 @@ GemmPlan gemm_plan(int M, int N, int K, int G) {
 // 153-157, down M = 2048 313 -> 308, against 1; 4 and 5 no better; same outputs bit for bit).
 constexpr int kWeightAhead = 3;
 
-// Tile plan of the packed-format GEMM (M > 16 through ns_w4_linear_packed). On MI355X (interleaved
-// A/B runs, us; the standard GEMM in brackets where the shape is a config-4 one):
-//  * 128 x 128 tiles, four workgroups per CU, when they make more than two rounds of the CUs
-//    (gate/up 37888 x 3584 at M = 512 133.0 [152.2], at M = 2048 476.3 [530.8]; qkv 4608 x 3584
-//    at M = 2048 77.4 against 81.3 split).
-//  * The same tiles with K split over two wave groups (one eight-wave workgroup, two per CU)
-//    when they make one to two rounds (down 3584 x 18944 at M = 2048: 266.2 [298.2], 300.5
-//    unsplit, 284.4 for 256 x 128 tiles split the same way; at short K too: qkv at M = 512 31.8
-//    against 39.4 unsplit, at M = 1024 49.6 against 54.1, 3584 x 3584 at M = 2048 57.0 against
-//    62.7, gate/up at M = 128 50.3 against 54.4).
-//  * 128 x 64 tiles with K split over four groups of two waves when 128 x 128 tiles would leave
-//    CUs idle and the 128 x 64 ones fill three quarters to all of them (down at M = 512: 98.8
-//    [102.3], 189.8 for 128 x 128 tiles; 3584 x 3584 at M = 512 24.1 against 31.4 split in two).
-//  * 64 x 64 tiles with K split over four groups of two waves, two per CU, on smaller grids
-//    (down at M = 256 57.7 against 89.3 for 128 x 64 tiles and 140.5 for the two-group split,
-//    64.6 for the standard GEMM; 3584 x 3584 at M = 256 15.4 against 22.4; qkv at M = 128 15.1
-//    against 22.4) and whenever M <= 64, where 128-row tiles would be half empty (gate/up at
-//    M = 32 33.7 against 49.7 for the two-group split).
+// Tile plans of the packed-format GEMM (M > 16 through ns_w4_linear_packed), as rows x columns and
+// wave groups that split K; plan numbers index kPkPlans. On MI355X (us):
+//  * A grid that fits the CUs once takes the smallest tiles that fit, as the standard GEMM's. Times
+//    of one round at K = 3584 / 18944: 64 x 64 14.4 / 57, 96 x 64 18.9 / 70, 128 x 64 20.5 / 87, 64 x
+//    128 21.5 / 99, 96 x 128 27 / 118, 128 x 128 31 / 133, 160 x 128 37 / 155, 192 x 128 43 / 175 (64 x
+//    128 ahead of 128 x 64 for short K: 2048 x 1536 at M = 850 11.8 against 14.6). Against 64 x 64,
+//    128 x 64 and 128 x 128 alone: 3584 x 18944 at M = 700 134 -> 123, M = 1200 209 -> 161; 4608 x 3584
+//    at M = 400 28.5 -> 22.3, M = 600 33.4 -> 27.1, M = 1000 51.4 -> 37.7. At short K the 160- and
+//    192-row tiles lose to two rounds (17920 x 1536 at M = 150: 27.7 against 25.2), so they need
+//    K >= 2048.
+//  * 64 x 64 tiles whenever M <= 64, where taller tiles would be half empty (gate/up at M = 32 33.7
+//    against 49.7 for 128 x 128).
+//  * 128 x 128 tiles, four four-wave workgroups per CU, when they make more than two rounds of the
+//    CUs (gate/up 37888 x 3584 at M = 512 133.0, 152.2 for the standard GEMM; at M = 2048 476.3 and
+//    530.8); the same tiles with K split over two wave groups (two eight-wave workgroups per CU) up
+//    to two rounds (3584 x 18944 at M = 2048 238 against 262, 3584 x 3584 50.2 against 53.7).
 // Weights one tile column (128 k) ahead in every plan: two columns ahead ran 3-8 % slower
 // (gate/up at M = 2048 489.6 against 473.0, M = 512 142.9 against 132.4), three 13 %.
+struct PkPlan {
+  int bm, bn;
+};
+constexpr PkPlan kPkPlans[] = {
+    {128, 128},  // 0: unsplit
+    {128, 128},  // 1: K split over 2 groups of four waves
+    {128, 64},   // 2: K split over 4 groups of two waves
+    {64, 64},    // 3: K split over 4 groups of two waves
+    {96, 64},    // 4: K split over 4 groups of two waves
+    {64, 128},   // 5: K split over 2 groups of four waves
+    {96, 128},   // 6: K split over 2 groups of four waves
+    {160, 128},  // 7: K split over 2 groups of four waves
+    {192, 128},  // 8: K split over 2 groups of four waves
+};
+
 int gemm_packed_plan(int M, int N, int K) {
-  (void)K;
   int cus = 256;  // the device's CU count (a failed query leaves MI355X's; the launch reports it)
   if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;
   if (M <= 64) return 3;
-  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  const long t128x64 = (long)((M + 127) / 128) * ((N + 63) / 64);
-  if (t128 < cus && 4 * t128x64 >= 3 * cus && t128x64 <= cus) return 2;
-  if (t128 > 2 * cus) return 0;
-  return 2 * t128 > cus ? 1 : 3;
+  auto count = [&](int p) { return (long)((M + kPkPlans[p].bm - 1) / kPkPlans[p].bm) * ((N + kPkPlans[p].bn - 1) / kPkPlans[p].bn); };
+  const int first = K >= 2048 ? 2 : 5, second = K >= 2048 ? 5 : 2;
+  for (const int p : {3, 4, first, second, 6, 1, 7, 8})
+    if (count(p) <= cus && (p < 7 || K >= 2048)) return p;
+  return count(0) > 2l * cus ? 0 : 1;
 }
 
 namespace {
 template <bool SW>
 hipError_t launch_gemm_packed_t(const uint16_t* A, const uint32_t* Wp, const uint16_t* Sp, uint16_t* C,
                                 int M, int N, int K, int plan, hipStream_t st) {
+  if (plan < 0 || plan >= (int)(sizeof(kPkPlans) / sizeof(kPkPlans[0]))) return hipErrorInvalidValue;
+  const dim3 grid((N + kPkPlans[plan].bn - 1) / kPkPlans[plan].bn, (M + kPkPlans[plan].bm - 1) / kPkPlans[plan].bm);
+#define NS_PK_CASE(P, BM, NWN, KS)                                                                     \
+  case P:                                                                                              \
+    static_assert(kPkPlans[P].bm == BM && kPkPlans[P].bn == 32 * NWN, "tile of the plan");             \
+    hipLaunchKernelGGL((w4_gemm_pk_kernel<BM, NWN, KS, 1, SW>), grid, dim3(64 * NWN * KS), 0, st, A, Wp, \
+                       Sp, C, M, N, K);                                                                \
+    return hipSuccess;
   switch (plan) {
-    case 0:  // 128 x 128 tiles
-      hipLaunchKernelGGL((w4_gemm_pk_kernel<128, 4, 1, 1, SW>), dim3((N + 127) / 128, (M + 127) / 128),
-                         dim3(256), 0, st, A, Wp, Sp, C, M, N, K);
-      return hipSuccess;
-    case 1:  // 128 x 128 tiles, K split over two groups of four waves
-      hipLaunchKernelGGL((w4_gemm_pk_kernel<128, 4, 2, 1, SW>), dim3((N + 127) / 128, (M + 127) / 128),
-                         dim3(512), 0, st, A, Wp, Sp, C, M, N, K);
-      return hipSuccess;
-    case 2:  // 128 x 64 tiles, K split over four groups of two waves
-      hipLaunchKernelGGL((w4_gemm_pk_kernel<128, 2, 4, 1, SW>), dim3((N + 63) / 64, (M + 127) / 128),
-                         dim3(512), 0, st, A, Wp, Sp, C, M, N, K);
-      return hipSuccess;
-    case 3:  // 64 x 64 tiles, K split over four groups of two waves
-      hipLaunchKernelGGL((w4_gemm_pk_kernel<64, 2, 4, 1, SW>), dim3((N + 63) / 64, (M + 63) / 64),
-                         dim3(512), 0, st, A, Wp, Sp, C, M, N, K);
-      return hipSuccess;
+    NS_PK_CASE(0, 128, 4, 1)
+    NS_PK_CASE(1, 128, 4, 2)
+    NS_PK_CASE(2, 128, 2, 4)
+    NS_PK_CASE(3, 64, 2, 4)
+    NS_PK_CASE(4, 96, 2, 4)
+    NS_PK_CASE(5, 64, 4, 2)
+    NS_PK_CASE(6, 96, 4, 2)
+    NS_PK_CASE(7, 160, 4, 2)
+    NS_PK_CASE(8, 192, 4, 2)
     default:
       return hipErrorInvalidValue;
   }
+#undef NS_PK_CASE
 }
 }  // namespace
 
@@ -1183,6 +1188,26 @@ hipError_t launch_gemm(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
       hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 4, false, 2>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
                          a.M, a.N, a.K, ilog2(a.G));
       return hipSuccess;
+    case 15:
+      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 2, 2, false, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 16:
+      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 17:
+      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 18:
+      hipLaunchKernelGGL((w4_gemm2_kernel<160, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 19:
+      hipLaunchKernelGGL((w4_gemm2_kernel<192, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
     default:
       return hipErrorInvalidValue;
   }
@@ -1234,6 +1259,26 @@ hipError_t launch_gemm_swiglu(const GemmArgs& a, const GemmPlan& p, hipStream_t 
     case 14:
       hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 4, true, 2>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
                          a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 15:
+      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 2, 2, true, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 16:
+      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 17:
+      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 18:
+      hipLaunchKernelGGL((w4_gemm2_kernel<160, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
+      return hipSuccess;
+    case 19:
+      hipLaunchKernelGGL((w4_gemm2_kernel<192, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
+                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
       return hipSuccess;
     default:
       return hipErrorInvalidValue;

@@ -26,9 +26,9 @@ def _deq(wq, s, G):
     return w.view(q.shape[0], -1)
 
 
-# (M, N, K, G): the 32 x 32, 32 x 64, 64 x 32, three-stage 32 x 64 and 64 x 128 plans at one row, at
-# their tile edges and past them, K whose blocks do not divide among the K groups, the plans above
-# them with ragged M, and the register-staged kernel (G = 96, K % 64 == 32)
+# (M, N, K, G): every tile plan with ragged M (32 to 192 rows, 32 to 128 columns, one round of the CUs
+# and several), at one row, at tile edges and past them, K whose blocks do not divide among the K
+# groups, and the register-staged kernel (G = 96, K % 64 == 32)
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,G", [
     (9, 128, 64, 64), (32, 256, 192, 64), (33, 1024, 704, 64), (65, 896, 1152, 128),
@@ -36,6 +36,9 @@ def _deq(wq, s, G):
     (200, 1536, 8960, 128), (250, 1024, 2048, 32), (17, 16384, 576, 64), (31, 9216, 1536, 128),
     (64, 17920, 1536, 128), (57, 16512, 448, 64), (100, 4608, 3584, 128), (129, 4608, 512, 128),
     (300, 3328, 1024, 128), (700, 1792, 896, 128), (1000, 8960, 256, 128), (2047, 18944, 128, 128),
+    (20, 17920, 448, 64), (40, 33024, 128, 128), (700, 3584, 384, 128), (1000, 4608, 192, 64),
+    (1200, 4608, 192, 32), (300, 12800, 128, 128), (1700, 3584, 8192, 128), (390, 3584, 8192, 128),
+    (500, 3584, 320, 64), (2000, 18944, 64, 64), (333, 8960, 320, 64), (1790, 3584, 8256, 64),
     (10, 128, 96, 96), (77, 256, 288, 96), (130, 384, 160, 32)])
 def test_linear_ragged_rows(kernels, M, N, K, G):
     wq, s = _weights(N, K, G, M + N)
@@ -85,11 +88,36 @@ def test_mlp_small_batch(kernels, M, N, K, G):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,G", [(9, 256, 256, 128), (40, 4608, 512, 128), (33, 17920, 256, 64),
                                      (100, 3584, 640, 32), (61, 18944, 128, 128), (200, 1536, 1920, 128),
-                                     (333, 8960, 256, 128), (900, 18944, 128, 128)])
+                                     (333, 8960, 256, 128), (900, 18944, 128, 128),
+                                     (20, 17920, 128, 128), (40, 33024, 128, 128), (300, 3328, 256, 128),
+                                     (700, 3584, 256, 128), (1000, 4608, 256, 128),
+                                     (1200, 4608, 256, 128), (500, 3584, 256, 128),
+                                     (390, 3584, 8192, 128), (1790, 3584, 8192, 128),
+                                     (1040, 18944, 64, 64)])
 def test_mlp_ragged_rows(kernels, M, N, K, G):
     wq, s = _weights(N, K, G, N + K)
     x = _x(M, K, M)
     assert torch.equal(kernels.w4_linear_swiglu(x, wq, s, G), _two_step(kernels, x, wq, s, G))
+
+
+# the packed GEMM's tile plans, ragged in M and N
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (17, 128, 128), (100, 896, 1024), (77, 200, 128), (260, 4096, 128), (410, 3584, 2048), (400, 3584, 128),
+    (500, 4608, 256), (700, 3504, 384), (333, 8960, 256), (1000, 4608, 2048), (1210, 4608, 2176),
+    (1900, 4608, 128), (350, 18944, 128), (700, 1800, 256), (1153, 3584, 2048)])
+def test_packed_ragged(kernels, M, N, K):
+    wq, s = _weights(N, K, 128, M + N)
+    wp, sp = kernels.w4_repack(wq, s)
+    x = _x(M, K, K)
+    y = kernels.w4_linear_packed(x, wp, sp, N)
+    ref = x.double() @ _deq(wq, s, 128).to(BF16).double().t()
+    err = (y.double() - ref).abs()
+    assert bool((err <= ref.abs() * 2.0 ** -8 + 2e-5 * ref.abs().max()).all())
+    if N % 16 == 0:
+        gu = y.view(M, N // 16, 2, 8)
+        two = kernels.swiglu(*(gu[:, :, i].reshape(M, N // 2).contiguous() for i in (0, 1)))
+        assert torch.equal(kernels.w4_linear_packed_swiglu(x, wp, sp, N), two)
 
 
 def test_rows_entry_points_reject():
