@@ -628,17 +628,21 @@ __global__ void __launch_bounds__(kAttnBlock)
 // the query heads, not the splits, so a long context (hundreds of splits) is merged by 56
 // workgroups of short loops (the earlier form, one workgroup per kv head walking every split,
 // took as long as the attention itself at 16384 cache rows).
+// LONG: the splits are attn_long_kernel's ranges (a template, so that the short form's chain from the
+// position to its loads stays as it is).
 constexpr int kMergeWaves = 8;
+template <bool LONG>
 __global__ void __launch_bounds__(kMergeWaves * kWave)
     decode_attn_merge_kernel(const float* __restrict__ opart, const float* __restrict__ ml,
                              const int* __restrict__ pos_p, uint16_t* __restrict__ out, int Hq,
-                             int max_len) {
+                             int max_len, int long_splits) {
   constexpr int D = kHeadDim;
   constexpr int SB = 16;  // splits per load batch of a wave
   __shared__ float red_m[kMergeWaves], red_l[kMergeWaves];
   __shared__ float red_o[kMergeWaves][kWave];
   const int n = min(*pos_p + 1, max_len);
-  const int nsplit = n > 0 ? (n + kChunk - 1) / kChunk : 0;
+  const int chunk = LONG ? long_chunk_rows(n, long_splits) : kChunk;  // rows per split
+  const int nsplit = n > 0 ? (n + chunk - 1) / chunk : 0;
   if (nsplit <= 1) return;  // written by the attention kernel itself
   const int h = blockIdx.x, lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -748,6 +752,10 @@ int attn_check(int Hq, int Hk, int D, int max_len, size_t work_bytes, const void
   return 0;
 }
 
+// Caches whose 128-row pieces of all kv heads outnumber the CUs are streamed (attn_long.hip), if the
+// launch merges. Either side of that line on MI355X, us with the merge (28 / 4, 12 / 2, 32 / 8 heads;
+// decode_attn_kernel first): 256 pieces 11.2 / 11.9, 11.6 / 12.0, 11.2 / 11.3; 512 pieces 16.8 / 14.5,
+// 18.6 / 14.7, 15.4 / 14.0.
 template <bool kFused>
 int launch_attn(const void* q, const void* bias, const void* inv_freq, void* kc, void* vc,
                 const int* pos, void* out, void* work, int Hq, int Hk, int max_len,
@@ -756,17 +764,31 @@ int launch_attn(const void* q, const void* bias, const void* inv_freq, void* kc,
   float* opart = static_cast<float*>(work);
   float* ml = opart + splits * Hq * kHeadDim;
   const float qscale = 1.4426950408889634f / sqrtf(static_cast<float>(kHeadDim));  // log2(e)/sqrt(D)
-  const dim3 grid(static_cast<unsigned>(splits), static_cast<unsigned>(Hk), 2u);
-  hipLaunchKernelGGL(decode_attn_kernel<kFused>, grid, dim3(kAttnBlock), 0, st,
-                     static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(bias),
-                     static_cast<const float*>(inv_freq), rot, static_cast<uint16_t*>(kc),
-                     static_cast<uint16_t*>(vc), pos, static_cast<uint16_t*>(out), opart, ml, Hq,
-                     Hk, max_len, qscale);
+  int cus = 256;  // the device's CU count (a failed query leaves MI355X's; the launch reports it)
+  if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;
+  const bool stream = merge && splits * Hk > static_cast<size_t>(cus);
+  if (stream) {
+    launch_attn_long(kFused, q, bias, inv_freq, kc, vc, pos, out, opart, ml, Hq, Hk, max_len, qscale, rot,
+                     st);
+  } else {
+    const dim3 grid(static_cast<unsigned>(splits), static_cast<unsigned>(Hk), 2u);
+    hipLaunchKernelGGL(decode_attn_kernel<kFused>, grid, dim3(kAttnBlock), 0, st,
+                       static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(bias),
+                       static_cast<const float*>(inv_freq), rot, static_cast<uint16_t*>(kc),
+                       static_cast<uint16_t*>(vc), pos, static_cast<uint16_t*>(out), opart, ml, Hq,
+                       Hk, max_len, qscale);
+  }
   if (merge && splits > 1) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return static_cast<int>(e);
-    hipLaunchKernelGGL(decode_attn_merge_kernel, dim3(Hq, kHeadDim / kWave), dim3(kMergeWaves * kWave),
-                       0, st, opart, ml, pos, static_cast<uint16_t*>(out), Hq, max_len);
+    const dim3 grid(Hq, kHeadDim / kWave), block(kMergeWaves * kWave);
+    const auto o = static_cast<uint16_t*>(out);
+    if (stream)
+      hipLaunchKernelGGL(decode_attn_merge_kernel<true>, grid, block, 0, st, opart, ml, pos, o, Hq, max_len,
+                         attn_long_splits(Hk, max_len));
+    else
+      hipLaunchKernelGGL(decode_attn_merge_kernel<false>, grid, block, 0, st, opart, ml, pos, o, Hq, max_len,
+                         0);
   }
   return last_status();
 }

@@ -6,15 +6,13 @@
 
 #include <algorithm>
 
+#include "attn_common.h"
 #include "internal_ops.h"
 #include "w4_common.h"
 #include "w4_kernels.h"
 
 namespace ns {
 namespace {
-
-typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------ bias + RoPE + KV append
 // Bound by launch and memory latency (1000 tokens of 36 heads: 9.5 us with the KV append, where
@@ -112,18 +110,6 @@ constexpr int kD = 128;
 constexpr int kRows = 128;    // query rows per workgroup
 constexpr int kKeys = 64;     // keys per block
 constexpr int kTile = kKeys * kD;  // bf16 elements of one K or V block
-
-__device__ __forceinline__ void attn_lds_load16(__amdgpu_buffer_rsrc_t r, uint16_t* dst, uint32_t voff,
-                                                uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff,
-                                           soff, 0, 0);
-}
-
-__device__ __forceinline__ u32x2_t lds_read_tr16(const uint16_t* p) {
-  return __builtin_bit_cast(
-      u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                   (__attribute__((address_space(3))) s16x4_t*)const_cast<uint16_t*>(p)));
-}
 
 struct AttnArgs {
   const uint16_t *q, *k, *v;

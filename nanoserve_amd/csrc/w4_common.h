@@ -29,6 +29,13 @@ constexpr int kStreamAux = 3;
 // activation load of the decode GEMV (w4_gemv.hip) reads the same split layout.
 constexpr int kAttnDecodeChunk = 128;
 
+// Cache rows per workgroup of the long-cache decode attention (attn_long.hip) at n rows and
+// `splits` workgroups per kv head, a multiple of kAttnDecodeChunk; its merge uses the same.
+__host__ __device__ inline int long_chunk_rows(int n, int splits) {
+  const int pieces = (n + kAttnDecodeChunk - 1) / kAttnDecodeChunk;
+  return (pieces + splits - 1) / splits * kAttnDecodeChunk;
+}
+
 // Workgroup barrier for LDS traffic: this wave's LDS operations complete (lgkmcnt(0)), then
 // s_barrier. Outstanding global loads and stores stay in flight; the release fence of
 // __syncthreads() would make a wave that has stored to global memory wait for every vector

@@ -87,6 +87,13 @@ hipError_t launch_gemv_m8_swiglu(const GemvArgs& a, hipStream_t st);
 // out [M][N/2] = bf16(silu(g) * u) of gu [M][N] with columns interleaved in blocks of 8.
 void launch_swiglu_interleaved(const uint16_t* gu, uint16_t* out, int M, int N, hipStream_t st);
 
+// Decode attention over a long cache (attn_long.hip): the partials of attn_long_splits(Hk, max_len)
+// ranges of long_chunk_rows rows, for decode_attn_merge_kernel (one range writes `out` itself).
+int attn_long_splits(int Hk, int max_len);
+void launch_attn_long(bool fused, const void* q, const void* bias, const void* inv_freq, void* k_cache,
+                      void* v_cache, const int* pos, void* out, float* opart, float* ml, int Hq, int Hk,
+                      int max_len, float qscale, const float* rot, hipStream_t st);
+
 struct GemmArgs {
   const uint16_t* A;   // X [M][K] bf16
   const uint32_t* Wq;  // [N][K/8]

@@ -128,3 +128,45 @@ def test_prompt_ops_reject_bad_arguments():
     assert qkv(P, None, P, P, P, 4, 4, 2, 128, 13, 16, None) == -2
     assert qkv(P, None, P, P, P, 4, 4, 2, 72, 0, 16, None) == -2
     assert qkv(P, P + 2, P, P, P, 4, 4, 2, 128, 0, 16, None) == -2
+
+
+# Caches past the streaming line (128-row pieces of all kv heads > CUs): positions at the edges of a
+# 16-row block, a 128-row piece and a workgroup's range, one range and many, empty waves and ranges
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hk,max_len", [(28, 4, 9000), (8, 8, 4200), (16, 16, 2200), (3, 1, 33000)])
+def test_decode_attention_streamed(kernels, Hq, Hk, max_len):
+    g = torch.Generator(device="cuda").manual_seed(Hq + max_len)
+    kc, vc = (torch.randn(Hk, max_len, 128, generator=g, device="cuda").to(BF16) for _ in range(2))
+    qkv = torch.randn((Hq + 2 * Hk) * 128, generator=g, device="cuda").to(BF16)
+    qkv[:Hq * 128] *= 3
+    b = torch.randn((Hq + 2 * Hk) * 128, generator=g, device="cuda").to(BF16)
+    inv = (1.0 / 1e6 ** (torch.arange(0, 128, 2).float() / 128)).cuda()
+    work = kernels.decode_attention_workspace(Hq, Hk, 128, max_len)
+    for pos in (0, 15, 16, 127, 128, 255, 1000, 2047, 2200 - 1, max_len // 2 + 1, max_len - 1, max_len + 5):
+        p = torch.tensor([pos], dtype=torch.int32, device="cuda")
+        k2, v2 = kc.clone(), vc.clone()
+        if pos + 1 < max_len:  # rows past the position must not matter
+            k2[:, pos + 1:] = float("nan")
+            v2[:, pos + 1:] = float("nan")
+        if pos < max_len:
+            k2[:, pos] = v2[:, pos] = float("nan")  # the token's own row is written by the call
+        got = kernels.decode_qkv_attention(qkv, b, inv, p, k2, v2, Hq, Hk, 128, work)
+        rot = torch.stack([torch.cos(pos * inv), torch.sin(pos * inv)])
+        ref = (qkv + b).clone()
+        kernels.decode_qkv(ref, None, inv, p, kc.clone(), vc.clone(), Hq, Hk, 128)
+        ref = ref.double().view(Hq + 2 * Hk, 1, 128)
+        n = min(pos + 1, max_len)
+        kk, vv = kc[:, :n].double(), vc[:, :n].double()
+        if pos < max_len:
+            kk[:, pos], vv[:, pos] = ref[Hq:Hq + Hk, 0], ref[Hq + Hk:, 0]
+            assert torch.equal(k2[:, pos].double(), kk[:, pos]) and torch.equal(v2[:, pos].double(), vv[:, pos])
+        q = ref[:Hq].transpose(0, 1).contiguous()
+        want = _ref(q, kk, vv, n - 1)
+        # half a bf16 ulp, the probabilities' two-term split and fp32 sums
+        bound = want.abs() * 2.0 ** -8 + 2.0 ** -14 * vv.abs().amax()
+        assert bool(((got.double() - want).abs() <= bound).all()), pos
+        plain = kernels.decode_attention(q.to(BF16).reshape(-1), k2, v2, p, Hq, Hk, 128, work)
+        assert torch.equal(plain, got), pos
+        if pos < max_len:  # an angle table gives the same angles' outputs
+            with_rot = kernels.decode_qkv_attention(qkv, b, inv, p, k2, v2, Hq, Hk, 128, work, rot=rot)
+            assert bool(((with_rot.double() - want).abs() <= 4 * bound + 1e-2).all()), pos
