@@ -497,7 +497,11 @@ class Qwen2Runner:
             act = gate_up_swiglu(h, li)
             # the down output joins the residual stream under the norm that follows this layer
             h = k.rmsnorm(x, lin(act, li, "wd"), self.norm_after[li], s.eps)
-        return F.linear(h[-1:] if last_only else h, self.lm_head)
+        if last_only:
+            h = h[-1:]
+        if h.shape[0] == 1 and s.hidden % 8 == 0 and s.hidden <= 8192:
+            return k.bf16_gemv(self.lm_head, x=h)  # 1.09 GB at 6.4 TB/s, against 4.6 for F.linear
+        return F.linear(h, self.lm_head)
 
     @torch.no_grad()
     def generate(self, prompt_ids, n_new: int, use_graph: bool = True):
