@@ -101,9 +101,9 @@ __global__ void __launch_bounds__(256)
 //  * LDS rows are 256 B (16 chunks of 16 B): K chunks are XOR-swizzled by row % 16 (the 16 rows of
 //    a fragment read hit distinct banks), V chunks by 4 (row % 4) (the 4-row x 64 B transpose
 //    reads spread over all banks).
-// MI355X, 28 / 4 heads: 1000 tokens from position 0 24.3 us (PyTorch's fused SDPA on repeated K / V
-// 67 us and its copies 40); 512 tokens after 3000 cached ones 52.5 + 8 us of merge (fp32 SDPA 682 us
-// and its copies 60).
+// MI355X, 28 / 4 heads: 1000 tokens from position 0 35.6 us with the merge (PyTorch's fused SDPA on repeated
+// K / V 67 us and its copies 40); 512 tokens after 3000 cached ones 53.3 us (fp32 SDPA 682 us and its
+// copies 60).
 //  * Few row tiles (short prompts, few kv heads) leave CUs idle: the keys are then split over
 //    blockIdx.z and a second kernel merges the fp32 partials.
 constexpr int kD = 128;
@@ -308,9 +308,11 @@ __global__ void __launch_bounds__(256) prompt_attn_merge_kernel(AttnArgs a) {
   const int id = blockIdx.x * 8 + (threadIdx.x >> 5), d = 4 * (threadIdx.x & 31);
   if (id >= all) return;
   float mx = -INFINITY;
+#pragma unroll 8
   for (int s = 0; s < a.splits; ++s) mx = fmaxf(mx, a.ml[2 * ((size_t)s * all + id)]);
   float l = 0.f;
   f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
   for (int s = 0; s < a.splits; ++s) {
     const size_t pr = (size_t)s * all + id;
     const float w = __builtin_amdgcn_exp2f(a.ml[2 * pr] - mx);
@@ -326,13 +328,16 @@ __global__ void __launch_bounds__(256) prompt_attn_merge_kernel(AttnArgs a) {
                                               pack_bf16x2_rne(o[2] * inv, o[3] * inv)};
 }
 
-// Splits over the keys: enough to give every CU two workgroups, each with at least four blocks.
+// Splits over the keys: enough for one and a half workgroups per CU, each with at least four blocks.
+// us (28 / 4 heads) for 1, 1.5, 2 and 3 per CU: 512 tokens at 3000 59.3, 53.3, 61.2, 61.7; 2000 tokens
+// at 0 60.1, 60.1, 72.6, 71.2; 200 at 4000 41.9, 38.6, 44.1, 43.1. With two blocks or one at least,
+// 20 tokens at 4000 take 30 and 39 us against 23.5, 200 at 0 14.3 and 13.7 against 10.2.
 int attn_splits(int T, int Hq, int Hk, int pos0) {
   int cus = 256;  // the device's CU count (a failed query leaves MI355X's; the launch reports it)
   if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;
   const long long tiles = (((long long)T * (Hq / Hk) + kRows - 1) / kRows) * Hk;
   const int blocks = (pos0 + T + kKeys - 1) / kKeys;
-  const long long want = (2 * cus + tiles - 1) / tiles;
+  const long long want = (3 * cus / 2 + tiles - 1) / tiles;
   return (int)std::max(1ll, std::min<long long>(want, blocks / 4));
 }
 
