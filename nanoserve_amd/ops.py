@@ -71,7 +71,15 @@ else:  # pragma: no cover - older torch builds
         return torch.cuda.current_stream(device).cuda_stream
 
 
+# The current device index without torch.cuda.current_device()'s initialisation check: every caller
+# has a GPU tensor in hand, so the runtime is initialised.
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def _require_gpu_tensor(t: torch.Tensor, name: str, dtype: torch.dtype) -> None:
+    # (the common case first: these checks run several times per launch, 0.3 us against 0.6 each)
+    if type(t) is torch.Tensor and t.is_cuda and t.dtype is dtype:
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.device.type != "cuda":
@@ -118,7 +126,7 @@ class Kernels:
     # handle (no Stream object per call: the eager launch path runs this for every operator)
     @staticmethod
     def _stream():
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+        return _raw_stream(_current_device())
 
     # reference ops.py:36-39
     @staticmethod
@@ -162,7 +170,7 @@ class Kernels:
         if M > 8 and M % 128:
             x = _aligned_rows(x)
         n = int(self.lib.ns_w4_linear_swiglu_rows_workspace(M, N, K, group))
-        y = torch.empty((M, I), dtype=torch.bfloat16, device=x.device) if out is None else out
+        y = x.new_empty((M, I)) if out is None else out
         tmp = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
         rc = self.lib.ns_w4_linear_swiglu_rows(
             x.data_ptr(), Wq.contiguous().data_ptr(), S.contiguous().data_ptr(), y.data_ptr(),
@@ -228,7 +236,7 @@ class Kernels:
                                  "no padding")
             y = out
         else:
-            y = torch.empty((max(M, 1), N), dtype=torch.bfloat16, device=x.device)
+            y = x.new_empty((M or 1, N))
         if work is not None:
             _require_gpu_tensor(work, "work", torch.uint8)
         if work is None or padded:
@@ -576,7 +584,7 @@ class Kernels:
         if Wp.shape[0] * 16 < N or Wp.shape[1] * 128 != K:
             raise ValueError("packed weights do not match N and x's K")
         if out is None:
-            out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+            out = x.new_empty((M, N))
         rc = self.lib.ns_w4_linear_packed(x.contiguous().data_ptr(), Wp.data_ptr(), Sp.data_ptr(),
                                           out.data_ptr(), M, N, K, group, self._stream())
         self._check(rc, "ns_w4_linear_packed")
