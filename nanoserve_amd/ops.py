@@ -190,7 +190,8 @@ class Kernels:
         N, K = W.shape
         if tuple(U.shape) != (K, K):
             raise ValueError(f"U must be [{K}, {K}], got {tuple(U.shape)}")
-        Wf = W.to(torch.float32).contiguous().clone()
+        # one copy, always the kernels' own (they overwrite it)
+        Wf = W.to(torch.float32, copy=True, memory_format=torch.contiguous_format)
         U = U.contiguous()
         Wq = torch.empty((N, K // 8), dtype=torch.int32, device=W.device)
         S = torch.empty((N, K // group), dtype=torch.bfloat16, device=W.device)
