@@ -419,11 +419,130 @@ __device__ __forceinline__ void k_group_handoff(V (&acc)[MI][NJ], float* lds, in
   }
 }
 
+// K-split handoff with the epilogue shared: every group adds up and stores one KS-th of its tile's
+// rows. own = part ks (E consecutive floats) of the accumulators x (KS E floats per lane, rows
+// ascending) summed over the groups in group order, through the free LDS ring `lds` (FLOATS
+// floats). With two groups each hands over the half that it does not keep; with more, every group
+// writes everything, so that no register is indexed by the group. Returns a slot of E * 64 floats
+// that nobody but this wave touches afterwards. Against handing everything to group 0, which then
+// works through the sums, the SwiGLU and the stores alone while the other waves have left (same
+// bits; us): 4608 x 3584 at M = 16 8.9 -> 8.3, M = 100 14.5 -> 13.8; 2048 x 1536 at M = 100 6.2 ->
+// 5.6; SwiGLU 17920 x 1536 at M = 100 20.6 -> 18.3, 3328 x 1024 at M = 256 10.0 -> 7.4, 15744 x 3584
+// at M = 256 42.6 -> 40.3.
+template <int KS, int NWN, int FLOATS, int E>
+__device__ __forceinline__ float* k_group_share(const float (&x)[KS * E], float (&own)[E], float* lds, int wv,
+                                                int ks, int lane) {
+  constexpr int V = E % 4 == 0 ? 4 : 2;  // floats per LDS access
+  typedef float vec_t __attribute__((ext_vector_type(V)));
+  static_assert(E % V == 0, "whole vectors");
+  constexpr int SLOT = E * kWave;  // one part of one wave
+  auto put = [&](float* p, const float* v) {
+#pragma unroll
+    for (int e = 0; e < E; e += V) {
+      vec_t t;
+#pragma unroll
+      for (int c = 0; c < V; ++c) t[c] = v[e + c];
+      *reinterpret_cast<vec_t*>(p + e * kWave + lane * V) = t;
+    }
+  };
+  if constexpr (KS == 2) {
+    static_assert(2 * NWN * SLOT <= FLOATS, "the handed halves fit the ring");
+    float give[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      own[e] = ks ? x[E + e] : x[e];
+      give[e] = ks ? x[e] : x[E + e];
+    }
+    put(lds + ((ks ^ 1) * NWN + wv) * SLOT, give);
+    lds_sync();
+    float* p = lds + (ks * NWN + wv) * SLOT;
+#pragma unroll
+    for (int e = 0; e < E; e += V) {
+      const vec_t t = *reinterpret_cast<const vec_t*>(p + e * kWave + lane * V);
+#pragma unroll
+      for (int c = 0; c < V; ++c) own[e + c] += t[c];
+    }
+    return p;
+  } else {
+    static_assert(KS * KS * NWN * SLOT <= FLOATS, "every group's accumulators fit the ring");
+#pragma unroll
+    for (int part = 0; part < KS; ++part) put(lds + ((ks * NWN + wv) * KS + part) * SLOT, &x[part * E]);
+    lds_sync();
+    float* p = lds + (wv * KS + ks) * SLOT;
+#pragma unroll
+    for (int g = 0; g < KS; ++g)
+#pragma unroll
+      for (int e = 0; e < E; e += V) {
+        const vec_t t =
+            *reinterpret_cast<const vec_t*>(p + g * NWN * KS * SLOT + e * kWave + lane * V);
+#pragma unroll
+        for (int c = 0; c < V; ++c) own[e + c] = g == 0 ? t[c] : own[e + c] + t[c];
+      }
+    return p;
+  }
+}
+
+// Row of value e of part ks inside the tile, before + 4 (lane / 32).
+template <int E>
+__device__ __forceinline__ int part_row(int ks, int e) {
+  return E >= 4 ? 2 * E * ks + 8 * (e >> 2) + (e & 3) : 8 * (ks >> 1) + 2 * (ks & 1) + e;
+}
+
+// Epilogue of one part of a wave's 32-column slice (k_group_share): E values per lane, rounded to
+// bf16, through the wave's LDS slot (row stride 32) and out as 16-byte row segments. Rows past M
+// and columns past N are not stored.
+template <int E>
+__device__ __forceinline__ void store_part(const float (&v)[E], uint16_t* lds, uint16_t* C, int M, int N,
+                                           int m0, int n0w, int ks, int lane) {
+  const int ln = lane & 31, kh = lane >> 5;
+  asm volatile("" ::: "memory");  // the slot's floats have been read
+#pragma unroll
+  for (int e = 0; e < E; e += 2) {
+    const int row = E >= 4 ? 8 * (e >> 2) + 4 * kh + (e & 3) : 2 * kh + e;  // row of the slot
+    const uint32_t pk = pack_bf16x2_rne(v[e], v[e + 1]);
+    lds[row * 32 + ln] = (uint16_t)pk;
+    lds[(row + 1) * 32 + ln] = (uint16_t)(pk >> 16);
+  }
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's rows are in LDS
+  asm volatile("" ::: "memory");
+  const int n = n0w + 8 * (lane & 3);
+#pragma unroll
+  for (int p = 0; p < (2 * E + 15) / 16; ++p) {
+    const int row = 16 * p + (lane >> 2);
+    const int m = m0 + (E >= 4 ? 2 * E * ks + row : part_row<E>(ks, 0) + 4 * (row >> 1) + (row & 1));
+    if (row < 2 * E && m < M) {
+      const u32x4_t t = *reinterpret_cast<const u32x4_t*>(&lds[row * 32 + 8 * (lane & 3)]);
+      if (n + 8 <= N) {
+        *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = t;
+      } else {
+        for (int c = 0; c < 8; ++c)
+          if (n + c < N) C[(size_t)m * N + n + c] = (uint16_t)(t[c >> 1] >> (16 * (c & 1)));
+      }
+    }
+  }
+}
+
+// SwiGLU epilogue of one part (store_tile_swiglu's pairing and rounding).
+template <int E>
+__device__ __forceinline__ void store_part_swiglu(const float (&v)[E], uint16_t* Y, int M, int N, int m0,
+                                                  int n0w, int ks, int lane) {
+  const int ln = lane & 31, kh = lane >> 5, n = n0w + ln, Nh = N >> 1;
+  const int o = ((n >> 4) << 3) + (n & 7);
+  const bool gate = (ln & 8) == 0 && n < N;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int m = m0 + part_row<E>(ks, e) + 4 * kh;
+    const float g = round_bf16(v[e]);
+    const float u = lane_xor8(g);
+    if (gate && m < M) Y[(size_t)m * Nh + o] = (uint16_t)f32_to_bf16_rne(silu_mul(g, u));
+  }
+}
+
 // KS > 1 (tile grids too small to fill the chip, e.g. down at M = 512): KS groups of NWN waves
 // split K inside the workgroup. Group ks computes 64-k blocks ks, ks + KS, ... into its own
 // accumulators through its own part of the LDS ring (step t loads and computes block t KS + ks
-// in every group); at the end groups 1 .. KS-1 hand their accumulators to group 0 through LDS,
-// and group 0 adds them in group order and stores the tile.
+// in every group); at the end each group adds up one KS-th of the tile's rows through LDS, in group
+// order, and stores it.
 // 256-row tiles carry 128 accumulators per lane: the launch bound asks for two waves per SIMD
 // (two four-wave workgroups per CU, or one eight-wave workgroup with KS = 2) so the compiler
 // keeps them in VGPRs beside the operands.
@@ -619,10 +738,17 @@ __global__ __launch_bounds__(NWN * KS * kWave, BM >= 256 && KS == 1 ? 2 : 1) voi
   wait_vmcnt_c<0>();  // the trailing out-of-range loads have landed before the LDS is reused
   lds_barrier();      // every wave is done reading the ring
   if constexpr (KS > 1) {
-    k_group_handoff<KS, NWN, sizeof(As) / 4>(acc, reinterpret_cast<float*>(As), wv, ks, lane);
-    if (ks != 0) return;  // no barrier follows
-  }
-  if constexpr (SW)
+    static_assert(WN == 32, "one 32-column fragment per wave");
+    constexpr int E = 16 * MI / KS;
+    float x[KS * E], own[E];
+#pragma unroll
+    for (int e = 0; e < KS * E; ++e) x[e] = acc[e / 16][0][e % 16];
+    float* slot = k_group_share<KS, NWN, sizeof(As) / 4, E>(x, own, reinterpret_cast<float*>(As), wv, ks, lane);
+    if constexpr (SW)
+      store_part_swiglu<E>(own, C, M, N, m0, n0 + wv * WN, ks, lane);
+    else
+      store_part<E>(own, reinterpret_cast<uint16_t*>(slot), C, M, N, m0, n0 + wv * WN, ks, lane);
+  } else if constexpr (SW)
     store_tile_swiglu<MI, NJ>(acc, C, M, N, m0, n0 + wv * WN);
   else if constexpr (kLdsEpilogue)
     store_tile_lds<MI, NJ, ELS>(acc, &As[wv * BM * ELS], C, M, N, m0, n0 + wv * WN);
@@ -696,8 +822,9 @@ __device__ __forceinline__ void store_tile_16x16_swiglu(const f32x4_t (&acc)[BM 
                     (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
   const int cr = lane >> 1, cc = lane & 1;
 #pragma unroll
-  for (int p = 0; p < BM / 32; ++p) {
+  for (int p = 0; p < (BM + 31) / 32; ++p) {
     const int row = 32 * p + cr;
+    if (BM % 32 != 0 && row >= BM) continue;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * 16 + 8 * cc]);
     const int m = m0 + row, o = o0 + 8 * cc;
     if (full) {
@@ -758,9 +885,9 @@ __device__ __forceinline__ uint32_t dequant_pair_bf16_pk(uint32_t w, uint32_t vm
 //    WD steps ahead are issued at the step's first block into a register ring of WD + 1 slots.
 //  * KS > 1 (tile grids that do not fill the chip, e.g. the 7B down projection): KS groups of
 //    NWN waves split the tile columns (group g takes columns g, g + KS, ..., through its own
-//    two stages); groups 1 .. KS-1 then hand their accumulators to group 0 through LDS, and
-//    group 0 adds them in group order.
-//  * Epilogue (group 0): each wave rounds its BM x 32 sub-tile to bf16 into a private part of
+//    two stages); the accumulators are then added in group order through LDS, by group 0 or in
+//    equal shares by every group.
+//  * Epilogue: each wave rounds its BM x 32 sub-tile to bf16 into a private part of
 //    the (then free) LDS ring and stores 16-byte row segments.
 template <int BM, int NWN, int KS, int WD, bool SW = false>
 __global__ __launch_bounds__(NWN * KS * kWave, KS > 1 ? 1 : 4)
@@ -938,7 +1065,26 @@ void w4_gemm_pk_kernel(const uint16_t* __restrict__ A, const uint32_t* __restric
   wait_vmcnt_c<0>();
   lds_barrier();  // every wave is done with the ring
 
-  if constexpr (KS > 1) {
+  // Four groups: each stores BM / 4 rows where those are whole fragments (4608 x 3584 at M = 100 14.1
+  // -> 12.6 us). Two groups keep the handoff to group 0: shared, the 128 x 128 kernel needs 134
+  // registers and loses its second workgroup per CU, or at 128 registers runs 1-2 % slower (3584 x
+  // 3584 at M = 2048 52.1 -> 53.0).
+  if constexpr (KS > 2 && BM / 16 % KS == 0) {
+    constexpr int E = BM / 2 / KS, BP = BM / KS;
+    float x[KS * E], own[E];
+    f32x4_t part[BP / 16][2];
+#pragma unroll
+    for (int e = 0; e < KS * E; ++e) x[e] = acc[e / 8][e / 4 % 2][e % 4];
+    float* slot = k_group_share<KS, NWN, sizeof(As) / 4, E>(x, own, reinterpret_cast<float*>(As), wv, ks, lane);
+    asm volatile("" ::: "memory");  // the slot's floats have been read
+#pragma unroll
+    for (int e = 0; e < E; ++e) part[e / 8][e / 4 % 2][e % 4] = own[e];
+    if constexpr (SW)
+      store_tile_16x16_swiglu<BP>(part, reinterpret_cast<uint16_t*>(slot), C, M, N, m0 + BP * ks, n0 + 32 * wv, lane);
+    else
+      store_tile_16x16<BP>(part, reinterpret_cast<uint16_t*>(slot), C, M, N, m0 + BP * ks, n0 + 32 * wv, lane);
+    return;
+  } else if constexpr (KS > 1) {
     k_group_handoff<KS, NWN, sizeof(As) / 4>(acc, reinterpret_cast<float*>(As), wv, ks, lane);
     if (ks != 0) return;  // no barrier follows
   }
@@ -996,10 +1142,10 @@ GemmPlan gemm_plan(int M, int N, int K, int G) {
     //  * A grid that fits the CUs once is bound by the time of one tile (its chain of loads over K,
     //    then the arithmetic of its CU): the plan with the smallest tiles that still fits, K split
     //    over as many wave groups as its LDS ring allows, with three blocks of activations in
-    //    flight for the smallest. Times of one round at K = 3584 / 18944, us: 32 x 32 9.9 / 42, 32 x
+    //    flight for the smallest. Times of one round at K = 3584 / 18944, us: 32 x 32 9.3 / 41, 32 x
     //    64 12.5 / 50, 64 x 32 13.7 / 54, 64 x 64 15.6 / 68, 96 x 64 19.5 / 82, 64 x 128 22 / 108,
     //    128 x 64 23 / 100, 96 x 128 29 / 134, 128 x 128 33 / 155, 160 x 128 38 / 185, 192 x 128 45 /
-    //    215; 64 x 128 and 128 x 64 change places at K = 8192 (two K groups against four).
+    //    215; 64 x 128 and 128 x 64 change places at K = 4096 (two K groups against four).
     //    Against the 64 x 64, 128 x 64 and 128 x 128 plans alone: 4608 x 3584 at M = 16 17.4 -> 9.6,
     //    M = 64 17.3 -> 13.4, M = 600 32.9 -> 29.6, M = 1000 49.4 -> 41.2; 3584 x 18944 at M = 64 71.2 ->
     //    42.0, M = 700 159 -> 137, M = 1200 237 -> 192; 1536 x 8960 at M = 100 35.1 -> 18.1, M = 700
@@ -1018,7 +1164,7 @@ GemmPlan gemm_plan(int M, int N, int K, int G) {
     //    M = 2048 590 -> 555 us; with fewer rounds (gate/up M = 512) 128 x 128 is faster.
     //  * 128 x 128 tiles, three workgroups per CU: the rest.
     auto count = [&](int c) { return (long)((M + kCfgs[c].bm - 1) / kCfgs[c].bm) * ((N + kCfgs[c].bn - 1) / kCfgs[c].bn); };
-    const int first = K >= 8192 ? 8 : 16, second = K >= 8192 ? 16 : 8;
+    const int first = K >= 4096 ? 8 : 16, second = K >= 4096 ? 16 : 8;
     int c = 0;
     for (const int p : {10, 11, 12, 9, 15, first, second, 17, 5, 18, 19})
       if (c == 0 && count(p) <= cus && (M > 64 || kCfgs[p].bm <= (M <= 32 ? 32 : 64))) c = p;
@@ -1058,14 +1204,16 @@ constexpr int kWeightAhead = 3;
 //    128 ahead of 128 x 64 for short K: 2048 x 1536 at M = 850 11.8 against 14.6). Against 64 x 64,
 //    128 x 64 and 128 x 128 alone: 3584 x 18944 at M = 700 134 -> 123, M = 1200 209 -> 161; 4608 x 3584
 //    at M = 400 28.5 -> 22.3, M = 600 33.4 -> 27.1, M = 1000 51.4 -> 37.7. At short K the 160- and
-//    192-row tiles lose to two rounds (17920 x 1536 at M = 150: 27.7 against 25.2), so they need
-//    K >= 2048.
+//    192-row tiles lose to two rounds, so they need K >= 1536; the 96 x 64 tiles need K >= 2048.
 //  * 64 x 64 tiles whenever M <= 64, where taller tiles would be half empty (gate/up at M = 32 33.7
 //    against 49.7 for 128 x 128).
 //  * 128 x 128 tiles, four four-wave workgroups per CU, when they make more than two rounds of the
 //    CUs (gate/up 37888 x 3584 at M = 512 133.0, 152.2 for the standard GEMM; at M = 2048 476.3 and
 //    530.8); the same tiles with K split over two wave groups (two eight-wave workgroups per CU) up
-//    to two rounds (3584 x 18944 at M = 2048 238 against 262, 3584 x 3584 50.2 against 53.7).
+//    to two rounds (3584 x 18944 at M = 2048 238 against 262, 3584 x 3584 50.2 against 53.7), unless
+//    96 x 128 tiles fit two rounds, both of a CU's workgroups resident (9984 x 2304 at M = 548 38.7 ->
+//    33.0, 5504 x 1792 at M = 676 27.9 -> 22.8). Over 1277 random shapes (M 65-2048, N 1024-25600, K
+//    896-18944) the rule is 0.7 % from the best plan of each shape.
 // Weights one tile column (128 k) ahead in every plan: two columns ahead ran 3-8 % slower
 // (gate/up at M = 2048 489.6 against 473.0, M = 512 142.9 against 132.4), three 13 %.
 struct PkPlan {
@@ -1088,10 +1236,10 @@ int gemm_packed_plan(int M, int N, int K) {
   if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;
   if (M <= 64) return 3;
   auto count = [&](int p) { return (long)((M + kPkPlans[p].bm - 1) / kPkPlans[p].bm) * ((N + kPkPlans[p].bn - 1) / kPkPlans[p].bn); };
-  const int first = K >= 2048 ? 2 : 5, second = K >= 2048 ? 5 : 2;
+  const int first = K >= 1536 ? 2 : 5, second = K >= 1536 ? 5 : 2;
   for (const int p : {3, 4, first, second, 6, 1, 7, 8})
-    if (count(p) <= cus && (p < 7 || K >= 2048)) return p;
-  return count(0) > 2l * cus ? 0 : 1;
+    if (count(p) <= cus && (p != 4 || K >= 2048) && (p < 7 || K >= 1536)) return p;
+  return count(6) <= 2l * cus ? 6 : count(0) > 2l * cus ? 0 : 1;
 }
 
 namespace {

@@ -105,7 +105,8 @@ def test_mlp_ragged_rows(kernels, M, N, K, G):
 @pytest.mark.parametrize("M,N,K", [
     (17, 128, 128), (100, 896, 1024), (77, 200, 128), (260, 4096, 128), (410, 3584, 2048), (400, 3584, 128),
     (500, 4608, 256), (700, 3504, 384), (333, 8960, 256), (1000, 4608, 2048), (1210, 4608, 2176),
-    (1900, 4608, 128), (350, 18944, 128), (700, 1800, 256), (1153, 3584, 2048)])
+    (1900, 4608, 128), (350, 18944, 128), (700, 1800, 256), (1153, 3584, 2048), (548, 9984, 256),
+    (155, 7536, 384), (806, 1536, 1920)])
 def test_packed_ragged(kernels, M, N, K):
     wq, s = _weights(N, K, 128, M + N)
     wp, sp = kernels.w4_repack(wq, s)
