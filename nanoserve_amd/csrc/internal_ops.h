@@ -38,8 +38,9 @@ size_t ns_prompt_attention_workspace(int T, int Hq, int Hk, int pos0);
  * reference uses PyTorch SDPA, python/nanoserve/qwen.py:124-133). Query t attends over keys
  * 0 .. pos0 + t. q: token stride q_stride, heads [Hq][128] contiguous; k, v: key j of kv head g
  * at g * kv_head_stride + j * kv_stride (strides in elements), 128 values each; out
- * [T][Hq * 128] bf16. Products of the bf16 operands and all sums in fp32, softmax in fp32, the
- * probabilities to 16 significant bits (two bf16 terms).
+ * [T][Hq * 128] bf16. Products of the bf16 operands and all sums in fp32, softmax in fp32; the
+ * probabilities enter the second product with all 24 bits of fp32 (three bf16 terms) for pos0 > 0
+ * and with 16 (two terms) for pos0 == 0.
  * -2 for Hq % Hk != 0, sizes <= 0, pos0 < 0, strides not a multiple of 8 or rows that reach
  * 2 GiB, NULL or pointers that are not 16-byte aligned, work_bytes too small.
  */

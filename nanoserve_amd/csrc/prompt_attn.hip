@@ -96,13 +96,17 @@ __global__ void __launch_bounds__(256)
 //    so the softmax needs one lane swap per reduction, and the score registers are, as they
 //    stand, the B operand of O^T = V^T P^T: lane half kh holds keys {4 kh + b, 8 + 4 kh + b} of each
 //    16, and ds_read_b64_tr_b16 delivers V^T's fragment for exactly those keys.
-//  * Probabilities enter the product as two bf16 terms, p = hi + lo (p - hi is exact in fp32): the
-//    result keeps fp32-like accuracy for a third more MFMAs.
+//  * Probabilities enter the product as bf16 terms, each the rounding of what the terms before it
+//    leave (exact in fp32). Prompts from position 0 take two (16 significant bits, where fused bf16
+//    attention holds 8). Chunks after cached positions take three, the whole fp32 probability, as an
+//    attention in fp32 holds it: with two, 0.23 % of the outputs are not the rounding of the float64
+//    result, with three 0.04 %, for fp32 SDPA 0.07 % (28 / 4 heads, 512 tokens at 3000; 62.6 us
+//    against 54.9 with two).
 //  * LDS rows are 256 B (16 chunks of 16 B): K chunks are XOR-swizzled by row % 16 (the 16 rows of
 //    a fragment read hit distinct banks), V chunks by 4 (row % 4) (the 4-row x 64 B transpose
 //    reads spread over all banks).
 // MI355X, 28 / 4 heads: 1000 tokens from position 0 35.6 us with the merge (PyTorch's fused SDPA on repeated
-// K / V 67 us and its copies 40); 512 tokens after 3000 cached ones 53.3 us (fp32 SDPA 682 us and its
+// K / V 67 us and its copies 40); 512 tokens after 3000 cached ones 62.6 us (fp32 SDPA 682 us and its
 // copies 60).
 //  * Few row tiles (short prompts, few kv heads) leave CUs idle: the keys are then split over
 //    blockIdx.z and a second kernel merges the fp32 partials.
@@ -119,6 +123,7 @@ struct AttnArgs {
   int T, R, Hk, pos0, splits;
 };
 
+template <int TERMS>
 __global__ void __launch_bounds__(256, 2) prompt_attn_kernel(AttnArgs a) {
   // one array per stage: a read of one stage then provably does not alias the loads in flight
   // into the other, so the compiler puts no wait for those before it
@@ -230,18 +235,21 @@ __global__ void __launch_bounds__(256, 2) prompt_attn_kernel(AttnArgs a) {
         for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
     }
     const float mc = m == -INFINITY ? 0.f : m * c;
-    u32x4_t ph[4], pl[4];  // B operands of the four 16-key steps
+    u32x4_t pt[TERMS][4];  // B operands of the four 16-key steps
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[t][r], c, -mc));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(s[t][r + 1], c, -mc));
+        float p0 = __builtin_amdgcn_exp2f(fmaf(s[t][r], c, -mc));
+        float p1 = __builtin_amdgcn_exp2f(fmaf(s[t][r + 1], c, -mc));
         l += p0 + p1;
-        const uint32_t hi = pack_bf16x2_rne(p0, p1);
-        ph[2 * t + (r >> 3)][(r & 7) >> 1] = hi;
-        pl[2 * t + (r >> 3)][(r & 7) >> 1] =
-            pack_bf16x2_rne(p0 - __uint_as_float(hi << 16), p1 - __uint_as_float(hi & 0xffff0000u));
+#pragma unroll
+        for (int i = 0; i < TERMS; ++i) {
+          const uint32_t term = pack_bf16x2_rne(p0, p1);
+          pt[i][2 * t + (r >> 3)][(r & 7) >> 1] = term;
+          p0 -= __uint_as_float(term << 16);
+          p1 -= __uint_as_float(term & 0xffff0000u);
+        }
       }
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -250,8 +258,9 @@ __global__ void __launch_bounds__(256, 2) prompt_attn_kernel(AttnArgs a) {
         const u32x2_t v0 = lds_read_tr16(&vb[vt[d] + 16 * t * kD]);
         const u32x2_t v1 = lds_read_tr16(&vb[vt[d] + (16 * t + 8) * kD]);
         const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, (u32x4_t){v0[0], v0[1], v1[0], v1[1]});
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, ph[t]), o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, pl[t]), o[d], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < TERMS; ++i)
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8_t, pt[i][t]), o[d], 0, 0, 0);
       }
   };
 
@@ -414,8 +423,11 @@ int ns_prompt_attention(const void* q, long long q_stride, const void* k, const 
   const unsigned tiles = (unsigned)((rows + ns::kRows - 1) / ns::kRows);
   if (tiles > 65535u) return -2;
   const auto st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(ns::prompt_attn_kernel, dim3((unsigned)Hk, tiles, (unsigned)a.splits), dim3(256),
-                     0, st, a);
+  const dim3 grid((unsigned)Hk, tiles, (unsigned)a.splits);
+  if (pos0 > 0)
+    hipLaunchKernelGGL(ns::prompt_attn_kernel<3>, grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(ns::prompt_attn_kernel<2>, grid, dim3(256), 0, st, a);
   if (a.splits > 1)
     hipLaunchKernelGGL(ns::prompt_attn_merge_kernel, dim3((unsigned)(((long long)rows * Hk + 7) / 8)),
                        dim3(256), 0, st, a);

@@ -45,11 +45,36 @@ def test_prompt_attention(kernels, T, pos0, Hq, Hk, cached):
     got = kernels.prompt_attention(q, k, v, Hq, pos0, work=work)
     again = kernels.prompt_attention(q, k, v, Hq, pos0, work=work)
     assert torch.equal(got, again)
-    # half a bf16 ulp of the result (at most 2^-8 of it), the probabilities' two-term split (2^-16
-    # of the values' magnitude) and fp32 sums
+    # half a bf16 ulp of the result (at most 2^-8 of it), the probabilities' split from position 0
+    # (2^-16 of the values' magnitude) and fp32 sums
     err = (got.double() - want).abs()
     bound = want.abs() * 2.0 ** -8 + 2.0 ** -14 * v[:, :n].double().abs().amax()
     assert bool((err <= bound).all()), float((err - bound).max())
+
+
+@pytest.mark.gpu
+def test_prompt_attention_keeps_fp32_probabilities(kernels):
+    """Behind cached positions the second product holds the whole fp32 probability: three keys whose
+    values cancel to about 2^-18 of them, so that an error of a probability is the result's error."""
+    Hk, T, pos0 = 16, 2, 3
+    g = torch.Generator(device="cuda").manual_seed(8)
+    # scores 0, about -0.5 and about -5 nats; the chunk's own keys score below -1000 (probability 0)
+    b = torch.tensor([0.0, -0.5, -5.0], device="cuda") * (1 + 0.3 * torch.rand(Hk, 3, generator=g, device="cuda"))
+    kk, v = (torch.zeros(Hk, pos0 + T, 128, dtype=BF16, device="cuda") for _ in range(2))
+    kk[:, :3, 0], kk[:, 3:, 0] = b.to(BF16), -1024.0
+    q = torch.zeros(T, Hk, 128, dtype=BF16, device="cuda")
+    q[..., 0] = 11.3125
+    p = torch.exp(kk[:, :3, :1].double() * 11.3125 / math.sqrt(128))
+    v[:, 1] = torch.randn(Hk, 128, generator=g, device="cuda").to(BF16)
+    v[:, 0] = -(p[:, 1] * v[:, 1].double()).to(BF16)
+    v[:, 2] = -((p[:, 1] * v[:, 1].double() + v[:, 0].double()) / p[:, 2]).to(BF16)
+    want = (p * v[:, :3].double()).sum(1) / p.sum(1)
+    work = kernels.prompt_attention_workspace(T, Hk, Hk, pos0)
+    got = kernels.prompt_attention(q.view(T, -1), kk, v, Hk, pos0, work=work).view(T, Hk, 128).double()
+    # exp2 and its argument to 2^-22 of the probability, a handful of fp32 sums, the result's bf16
+    # rounding; a probability of 16 bits is up to 2^-18 off
+    bound = 2.0 ** -20 * (p[:, 1] * v[:, 1].double()).abs() + 2.0 ** -8 * want.abs() + 1e-9
+    assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
 
 
 @pytest.mark.gpu
