@@ -166,14 +166,15 @@ class Kernels:
                 raise ValueError(f"out must be a contiguous tensor of shape {(M, I)}")
         if M == 0:
             return out if out is not None else x.new_empty((0, I))
-        x = x.contiguous()
+        # (names for the copies: an address whose copy is gone may already be another copy's)
+        x, Wq, S = x.contiguous(), Wq.contiguous(), S.contiguous()
         if M > 8 and M % 128:
             x = _aligned_rows(x)
         n = int(self.lib.ns_w4_linear_swiglu_rows_workspace(M, N, K, group))
         y = x.new_empty((M, I)) if out is None else out
         tmp = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
         rc = self.lib.ns_w4_linear_swiglu_rows(
-            x.data_ptr(), Wq.contiguous().data_ptr(), S.contiguous().data_ptr(), y.data_ptr(),
+            x.data_ptr(), Wq.data_ptr(), S.data_ptr(), y.data_ptr(),
             None if tmp is None else tmp.data_ptr(), n, M, N, K, group, self._stream())
         self._check(rc, "ns_w4_linear_swiglu")
         return y
@@ -263,10 +264,10 @@ class Kernels:
         if r is not None:
             _require_gpu_tensor(r, "r", torch.bfloat16)
             r = r.contiguous()
+        w = w.contiguous()
         y = torch.empty_like(x) if out is None else _check_out(out, x)
-        rc = self.lib.ns_rmsnorm(x.data_ptr(), None if r is None else r.data_ptr(),
-                                 w.contiguous().data_ptr(), y.data_ptr(), x.shape[0], x.shape[1],
-                                 eps, self._stream())
+        rc = self.lib.ns_rmsnorm(x.data_ptr(), None if r is None else r.data_ptr(), w.data_ptr(),
+                                 y.data_ptr(), x.shape[0], x.shape[1], eps, self._stream())
         self._check(rc, "ns_rmsnorm")
         return y
 
@@ -279,9 +280,9 @@ class Kernels:
         for t, n in ((q, "q"), (k, "k")):
             if t.stride(-1) != 1:
                 raise ValueError(f"{n} rows must be contiguous")
-        rc = self.lib.ns_rope(q.data_ptr(), k.data_ptr(), inv_freq.contiguous().data_ptr(),
-                              q.shape[0], n_heads, n_kv_heads, head_dim, pos0, q.stride(0),
-                              k.stride(0), self._stream())
+        inv_freq = inv_freq.contiguous()
+        rc = self.lib.ns_rope(q.data_ptr(), k.data_ptr(), inv_freq.data_ptr(), q.shape[0], n_heads,
+                              n_kv_heads, head_dim, pos0, q.stride(0), k.stride(0), self._stream())
         self._check(rc, "ns_rope")
 
     def swiglu(self, gate, up, out=None):
@@ -568,8 +569,9 @@ class Kernels:
         NT, C = (N + 15) // 16, K // 128
         Wp = torch.empty((NT, C, 256), dtype=torch.int32, device=Wq.device)
         Sp = torch.empty((NT, C, 16), dtype=torch.bfloat16, device=Wq.device)
-        rc = self.lib.ns_w4_repack(Wq.contiguous().data_ptr(), S.contiguous().data_ptr(),
-                                   Wp.data_ptr(), Sp.data_ptr(), N, K, group, self._stream())
+        Wq, S = Wq.contiguous(), S.contiguous()
+        rc = self.lib.ns_w4_repack(Wq.data_ptr(), S.data_ptr(), Wp.data_ptr(), Sp.data_ptr(), N, K,
+                                   group, self._stream())
         self._check(rc, "ns_w4_repack")
         return Wp, Sp
 
@@ -586,8 +588,9 @@ class Kernels:
             raise ValueError("packed weights do not match N and x's K")
         if out is None:
             out = x.new_empty((M, N))
-        rc = self.lib.ns_w4_linear_packed(x.contiguous().data_ptr(), Wp.data_ptr(), Sp.data_ptr(),
-                                          out.data_ptr(), M, N, K, group, self._stream())
+        x = x.contiguous()
+        rc = self.lib.ns_w4_linear_packed(x.data_ptr(), Wp.data_ptr(), Sp.data_ptr(), out.data_ptr(),
+                                          M, N, K, group, self._stream())
         self._check(rc, "ns_w4_linear_packed")
         return out
 
@@ -603,9 +606,9 @@ class Kernels:
             raise ValueError("packed weights do not match N and x's K")
         if out is None:
             out = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
-        rc = self.lib.ns_w4_linear_packed_swiglu(x.contiguous().data_ptr(), Wp.data_ptr(),
-                                                 Sp.data_ptr(), out.data_ptr(), M, N, K, group,
-                                                 self._stream())
+        x = x.contiguous()
+        rc = self.lib.ns_w4_linear_packed_swiglu(x.data_ptr(), Wp.data_ptr(), Sp.data_ptr(),
+                                                 out.data_ptr(), M, N, K, group, self._stream())
         self._check(rc, "ns_w4_linear_packed_swiglu")
         return out
 
