@@ -28,6 +28,12 @@ int ns_prompt_qkv(void* qkv, const void* bias, const void* inv_freq, void* k_cac
                   void* stream);
 
 /*
+ * 1 if ns_prompt_attention takes these sizes with keys kv_stride elements apart (its size limits: keys
+ * whose rows reach 2 GiB and more than 65535 tiles of 128 query rows per kv head are refused), else 0.
+ */
+int ns_prompt_attention_fits(int T, int Hq, int Hk, int pos0, long long kv_stride);
+
+/*
  * Bytes of workspace ns_prompt_attention uses for these sizes (fp32 partials of the splits over
  * the keys); 0 when the queries alone fill the GPU and nothing is split, or for invalid sizes.
  */
@@ -41,8 +47,7 @@ size_t ns_prompt_attention_workspace(int T, int Hq, int Hk, int pos0);
  * [T][Hq * 128] bf16. Products of the bf16 operands and all sums in fp32, softmax in fp32; the
  * probabilities enter the second product with all 24 bits of fp32 (three bf16 terms) for pos0 > 0
  * and with 16 (two terms) for pos0 == 0.
- * -2 for Hq % Hk != 0, sizes <= 0, pos0 < 0, strides not a multiple of 8 or rows that reach
- * 2 GiB, NULL or pointers that are not 16-byte aligned, work_bytes too small.
+ * -2 where ns_prompt_attention_fits is 0, for strides that are not a multiple of 8, NULL or pointers that are not 16-byte aligned, work_bytes too small.
  */
 int ns_prompt_attention(const void* q, long long q_stride, const void* k, const void* v,
                         long long kv_stride, long long kv_head_stride, void* out, void* work,

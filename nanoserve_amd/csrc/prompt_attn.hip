@@ -357,6 +357,16 @@ bool attn_sizes_ok(int T, int Hq, int Hk, int pos0) {
          (long long)pos0 + T < (1ll << 30) && (long long)T * Hq < (1ll << 30);
 }
 
+unsigned attn_row_tiles(int T, int R) { return (unsigned)((T * R + kRows - 1) / kRows); }
+
+// The kernel's offsets and grid: block offsets past the last key stay below 2^32 and the range of the
+// keys' rows below 2^31; row tiles are a grid dimension.
+bool attn_fits(int T, int Hq, int Hk, int pos0, long long kv_stride) {
+  return attn_sizes_ok(T, Hq, Hk, pos0) && kv_stride >= kD && kv_stride < (1ll << 30) &&
+         ((long long)pos0 + T + 2 * kKeys) * kv_stride * 2 < (1ll << 31) &&
+         attn_row_tiles(T, Hq / Hk) <= 65535u;
+}
+
 }  // namespace
 }  // namespace ns
 
@@ -382,6 +392,10 @@ int ns_prompt_qkv(void* qkv, const void* bias, const void* inv_freq, void* k_cac
   return static_cast<int>(hipGetLastError());
 }
 
+int ns_prompt_attention_fits(int T, int Hq, int Hk, int pos0, long long kv_stride) {
+  return ns::attn_fits(T, Hq, Hk, pos0, kv_stride);
+}
+
 size_t ns_prompt_attention_workspace(int T, int Hq, int Hk, int pos0) {
   if (!ns::attn_sizes_ok(T, Hq, Hk, pos0)) return 0;
   const size_t splits = static_cast<size_t>(ns::attn_splits(T, Hq, Hk, pos0));
@@ -391,14 +405,12 @@ size_t ns_prompt_attention_workspace(int T, int Hq, int Hk, int pos0) {
 int ns_prompt_attention(const void* q, long long q_stride, const void* k, const void* v,
                         long long kv_stride, long long kv_head_stride, void* out, void* work,
                         size_t work_bytes, int T, int Hq, int Hk, int pos0, void* stream) {
-  if (!ns::attn_sizes_ok(T, Hq, Hk, pos0)) return -2;
+  if (!ns::attn_fits(T, Hq, Hk, pos0, kv_stride)) return -2;
   if (!q || !k || !v || !out) return -2;
   if (!ns::aligned(q, 16) || !ns::aligned(k, 16) || !ns::aligned(v, 16) || !ns::aligned(out, 16))
     return -2;
   if (q_stride % 8 || kv_stride % 8 || kv_head_stride % 8) return -2;
-  if (q_stride < (long long)Hq * ns::kD || kv_stride < ns::kD || kv_head_stride < 0) return -2;
-  // block offsets past the last key stay below 2^32 and the range below 2^31
-  if (((long long)pos0 + T + 2 * ns::kKeys) * kv_stride * 2 >= (1ll << 31)) return -2;
+  if (q_stride < (long long)Hq * ns::kD || kv_head_stride < 0) return -2;
   ns::AttnArgs a{};
   a.splits = ns::attn_splits(T, Hq, Hk, pos0);
   if (a.splits > 1) {
@@ -420,10 +432,8 @@ int ns_prompt_attention(const void* q, long long q_stride, const void* k, const 
   a.Hk = Hk;
   a.pos0 = pos0;
   const int rows = T * a.R;
-  const unsigned tiles = (unsigned)((rows + ns::kRows - 1) / ns::kRows);
-  if (tiles > 65535u) return -2;
   const auto st = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)Hk, tiles, (unsigned)a.splits);
+  const dim3 grid((unsigned)Hk, ns::attn_row_tiles(T, a.R), (unsigned)a.splits);
   if (pos0 > 0)
     hipLaunchKernelGGL(ns::prompt_attn_kernel<3>, grid, dim3(256), 0, st, a);
   else

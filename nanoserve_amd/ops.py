@@ -58,6 +58,7 @@ INTERNAL_SIGNATURES = {
     "ns_w4_linear_rows": [_VP] * 4 + [_I32] * 4 + [_VP],
     "ns_w4_linear_swiglu_rows_workspace": [_I32] * 4,
     "ns_w4_linear_swiglu_rows": [_VP] * 5 + [_SZ] + [_I32] * 4 + [_VP],
+    "ns_prompt_attention_fits": [_I32] * 4 + [_I64],
     "ns_prompt_attention_workspace": [_I32] * 4,
     "ns_prompt_attention": [_VP, _I64, _VP, _VP, _I64, _I64, _VP, _VP, _SZ, _I32, _I32, _I32, _I32,
                             _VP],
@@ -525,6 +526,10 @@ class Kernels:
                                     pos0, 0 if k_cache is None else k_cache.shape[1],
                                     self._stream())
         self._check(rc, "ns_prompt_qkv")
+
+    def prompt_attention_fits(self, T, n_heads, n_kv_heads, pos0, kv_stride):
+        """Whether prompt_attention takes these sizes with keys kv_stride elements apart."""
+        return bool(self.lib.ns_prompt_attention_fits(T, n_heads, n_kv_heads, pos0, kv_stride))
 
     def prompt_attention_workspace(self, T, n_heads, n_kv_heads, pos0, device=None):
         """A uint8 device tensor of the workspace prompt_attention uses for these sizes, or None.

@@ -396,12 +396,12 @@ class Qwen2Runner:
             self.packed.append(P)
         return self
 
-    def _prompt_attention_kernel_ok(self, T, pos0):
-        """Whether ns_prompt_attention takes this chunk: head size 128, and its 32-bit offsets
-        (keys in the cache rows or, without a cache, in the projection's rows; row tiles)."""
+    def _prompt_attention_kernel_ok(self, T, pos0, cached):
+        """Whether ns_prompt_attention takes this chunk: head size 128, and its limits over the rows
+        that hold the keys (the cache's or, without a cache, the projection's)."""
         s = self.shape
-        return (s.head_dim == 128 and (pos0 + T + 128) * s.qkv_rows * 2 < 1 << 31
-                and T * (s.heads // s.kv_heads) < 1 << 23)
+        return s.head_dim == 128 and self.k.prompt_attention_fits(
+            T, s.heads, s.kv_heads, pos0, s.head_dim if cached else s.qkv_rows)
 
     def _prompt_attention(self, q, k, v, pos0, li):
         """Causal attention of T query tokens at positions pos0 .. pos0+T-1 over cache / prompt
@@ -473,7 +473,7 @@ class Qwen2Runner:
             return k.w4_linear_swiglu(a, *self.layers[li]["wgu"], G)
 
         cached = use_cache or pos0 > 0
-        in_kernel = self._prompt_attention_kernel_ok(T, pos0)
+        in_kernel = self._prompt_attention_kernel_ok(T, pos0, cached)
         # one workspace for the pass: the layers' launches follow each other on one stream
         work = (k.prompt_attention_workspace(T, s.heads, s.kv_heads, pos0, device=self.dev)
                 if in_kernel else None)

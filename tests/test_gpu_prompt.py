@@ -155,6 +155,35 @@ def test_prompt_ops_reject_bad_arguments():
     assert qkv(P, P + 2, P, P, P, 4, 4, 2, 128, 0, 16, None) == -2
 
 
+def test_prompt_attention_limits_follow_the_key_rows():
+    """The runner's choice of the kernel is the kernel's own rule: 32-bit offsets over the rows the keys
+    lie in (128 values in a cache, the projection's width without one) and 65535 row tiles."""
+    from nanoserve_amd import Kernels
+    from nanoserve_amd.qwen import Qwen2Runner, Qwen2Shape
+
+    r = Qwen2Runner.__new__(Qwen2Runner)
+    r.k, r.shape = Kernels(), Qwen2Shape(layers=1, hidden=3584, heads=28, kv_heads=4)
+    P = 0x10000
+
+    def ok(T, pos0, cached):
+        fits = r._prompt_attention_kernel_ok(T, pos0, cached)
+        stride = 128 if cached else r.shape.qkv_rows
+        if not fits:  # refused before any launch
+            assert r.k.lib.ns_prompt_attention(P, r.shape.qkv_rows, P, P, stride, 128, P, P, 1 << 62, T,
+                                               28, 4, pos0, None) == -2
+        return fits
+
+    assert ok(512, 3000, True) and ok(512, 0, False)
+    assert ok(512, 300000, True) and ok(512, (1 << 23) - 641, True)
+    assert not ok(512, (1 << 23) - 640, True)
+    assert ok(232000, 0, False) and not ok(233000, 0, False)
+    # 7 heads per kv head: 65535 * 128 / 7 = 1198354.3 tokens
+    assert ok(1198354, 0, True) and not ok(1198355, 0, True) and not ok(1198372, 0, True)
+    assert not ok(0, 0, True) and not ok(1 << 30, 0, True)
+    r.shape = Qwen2Shape(layers=1, hidden=1024, heads=16, kv_heads=16, head_dim=64)
+    assert not r._prompt_attention_kernel_ok(512, 0, True)
+
+
 # Caches past the streaming line (128-row pieces of all kv heads > CUs): positions at the edges of a
 # 16-row block, a 128-row piece and a workgroup's range, one range and many, empty waves and ranges
 @pytest.mark.gpu
