@@ -116,6 +116,13 @@ def _plain_rope_theta(cfg) -> float:
     return float(next((b for b in bases if b), 10000.0))
 
 
+def _kernel_operand(t: torch.Tensor, shape) -> bool:
+    """Whether the one-launch operators of the prompt pass take this bias or output head: bf16,
+    contiguous, 16-byte aligned. PyTorch's operators take the others."""
+    return (t.dtype is torch.bfloat16 and t.shape == shape and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
 def _calibration_hessians(hf_model, calib_ids: torch.Tensor) -> dict:
     """Run the HF model on calib_ids and return {(layer, stack): H} with H = 2 X^T X / T
     (float64, on the model's device) of the inputs X of each stack of linear layers that share
@@ -481,6 +488,9 @@ class Qwen2Runner:
         def attention(qkv, bias, li):
             """Bias, RoPE, KV append and attention of the fused projection's output."""
             caches = (self.cache_k[li], self.cache_v[li]) if cached else (None, None)
+            if bias is not None and not _kernel_operand(bias, (s.qkv_rows,)):
+                qkv += bias
+                bias = None
             k.prompt_qkv(qkv, bias, self.inv_freq, s.heads, s.kv_heads, D, pos0, *caches)
             q, kk, v = qkv[:, :qn], qkv[:, qn:qn + kn], qkv[:, qn + kn:]
             if not in_kernel:
@@ -499,7 +509,8 @@ class Qwen2Runner:
             h = k.rmsnorm(x, lin(act, li, "wd"), self.norm_after[li], s.eps)
         if last_only:
             h = h[-1:]
-        if h.shape[0] == 1 and s.hidden % 8 == 0 and s.hidden <= 8192:
+        if (h.shape[0] == 1 and s.hidden % 8 == 0 and s.hidden <= 8192
+                and _kernel_operand(self.lm_head, (self.lm_head.shape[0], s.hidden))):
             return k.bf16_gemv(self.lm_head, x=h)  # 1.09 GB at 6.4 TB/s, against 4.6 for F.linear
         return F.linear(h, self.lm_head)
 
