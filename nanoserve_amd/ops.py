@@ -109,6 +109,12 @@ def _aligned_rows(x: torch.Tensor) -> torch.Tensor:
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two contiguous tensors share memory."""
+    pa, pb = a.data_ptr(), b.data_ptr()
+    return pa < pb + b.nbytes and pb < pa + a.nbytes
+
+
 class Kernels:
     """W4A16 kernels through the C ABI. ``path`` defaults to the in-tree library."""
 
@@ -172,13 +178,17 @@ class Kernels:
         if M > 8 and M % 128:
             x = _aligned_rows(x)
         n = int(self.lib.ns_w4_linear_swiglu_rows_workspace(M, N, K, group))
-        y = x.new_empty((M, I)) if out is None else out
+        # one launch reads x while it writes y: out may lie over x only through a tensor of its own
+        # (M = 1 and multiples of 128 are the callers' to keep apart)
+        y = out
+        if out is None or (M > 1 and M % 128 and _overlap(out, x)):
+            y = x.new_empty((M, I))
         tmp = torch.empty(n, dtype=torch.uint8, device=x.device) if n else None
         rc = self.lib.ns_w4_linear_swiglu_rows(
             x.data_ptr(), Wq.data_ptr(), S.data_ptr(), y.data_ptr(),
             None if tmp is None else tmp.data_ptr(), n, M, N, K, group, self._stream())
         self._check(rc, "ns_w4_linear_swiglu")
-        return y
+        return y if out is None or y is out else out.copy_(y)
 
     def w4_gptq(self, W, U, group=128):
         """Calibrated quantization (not in the reference, whose README.md:233-235 names it as

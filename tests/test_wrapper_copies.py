@@ -1,5 +1,6 @@
-"""Strided arguments of the Kernels wrappers: a contiguous copy must live until the launch has been
-issued (an address read from a copy that is already gone can belong to the next copy)."""
+"""What the Kernels wrappers hand to the library for strided and overlapping arguments: a contiguous
+copy must live until the launch has been issued (an address read from a copy that is already gone can
+belong to the next copy), and a launch must not write where it still reads."""
 import weakref
 
 import pytest
@@ -20,6 +21,7 @@ class _Lib:
         def call(*args):
             if not name.endswith("_workspace"):
                 self.launches.append((name, len(self.copies), all(c() is not None for c in self.copies)))
+                self.args = args
             return 0
 
         return call
@@ -67,6 +69,26 @@ def test_copies_outlive_the_launch(stub, call, copies):
     assert [(n, alive) for _, n, alive in stub.lib.launches] == [(copies, True)]
 
 
+# rows for which the activation was padded or the activation function ran as a launch of its own
+@pytest.mark.parametrize("M", [2, 5, 8, 9, 100, 130])
+@pytest.mark.parametrize("shift", [0, 128, -128])
+def test_swiglu_over_its_input(stub, M, shift):
+    wq, s = torch.ones(512, 32, dtype=torch.int32), torch.ones(512, 2, dtype=BF16)
+    buf = torch.ones(M * 256 + 256, dtype=BF16)
+    x, out = (buf[o:o + M * 256].view(M, 256) for o in (128, 128 + shift))
+    got = stub.w4_linear_swiglu(x, wq, s, out=out)
+    y = stub.lib.args[3]
+    assert got is out and (y + out.nbytes <= x.data_ptr() or y >= x.data_ptr() + x.nbytes)
+
+
+@pytest.mark.parametrize("M", [1, 4, 100, 128])
+def test_swiglu_writes_out_in_place(stub, M):
+    wq, s = torch.ones(512, 32, dtype=torch.int32), torch.ones(512, 2, dtype=BF16)
+    out = torch.ones(M, 256, dtype=BF16)
+    assert stub.w4_linear_swiglu(torch.ones(M, 256, dtype=BF16), wq, s, out=out) is out
+    assert stub.lib.args[3] == out.data_ptr()
+
+
 # scales above 1 MiB, so that the allocator serves them from the blocks it serves the codes from
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 4, 8, 20, 128])
@@ -81,5 +103,9 @@ def test_strided_weights(kernels, M):
     assert not wq.is_contiguous() and not s.is_contiguous()
     assert torch.equal(kernels.w4_linear(x, wq, s), kernels.w4_linear(x, wc, sc))
     assert torch.equal(kernels.w4_linear_swiglu(x, wq, s), kernels.w4_linear_swiglu(x, wc, sc))
+    y = kernels.w4_linear_swiglu(x, wc[:2 * K], sc[:2 * K])
+    if M not in (1, 128):  # out over the input
+        z = x.clone()
+        assert torch.equal(kernels.w4_linear_swiglu(z, wc[:2 * K], sc[:2 * K], out=z), y)
     for a, b in zip(kernels.w4_repack(wq, s), kernels.w4_repack(wc, sc)):
         assert torch.equal(a, b)
