@@ -109,6 +109,48 @@ def test_gptq_long_rows_sampled(k):
     assert np.array_equal(Wq[rows], Wq_o)
 
 
+def _factor(K, seed, exponents):
+    """A dense upper factor whose row i is scaled by 2^exponents[i]; off-diagonal entries are small
+    enough that a row's updates stay within a few times its weights."""
+    g = torch.Generator().manual_seed(seed)
+    U = torch.triu(torch.randn(K, K, generator=g) * 0.04, 1)
+    U += torch.diag(torch.empty(K).uniform_(0.5, 2.0, generator=g))
+    return torch.ldexp(U, exponents.view(K, 1))
+
+
+# Outside the range of the reciprocals (scales and diagonals past 2^+-60) and at its edges, updates and
+# weights that are subnormal, columns far past the clamp, NaN and infinite rows; row counts that are no
+# multiple of a panel's 16 or a tile's 128 rows
+@pytest.mark.parametrize("N,K", [(23, 128), (140, 384)])
+@pytest.mark.parametrize("what", ["scales", "diagonals", "both", "subnormal", "outliers", "special"])
+def test_gptq_guarded_divisions(k, N, K, what):
+    g = torch.Generator().manual_seed(N + K)
+    W = torch.randn(N, K, generator=g)
+    ex = torch.zeros(K, dtype=torch.int32)
+    if what in ("scales", "both"):  # rows from 2^-100 to 2^100, through every guard
+        W = torch.ldexp(W, torch.linspace(-100, 100, N).int().view(N, 1))
+    if what in ("diagonals", "both"):
+        ex = torch.linspace(-70, 70, K).int()[torch.randperm(K, generator=g)]
+    if what == "both":  # errors e = w / U and their products with U stay finite
+        W, ex = torch.ldexp(W, torch.full((1,), -20)), ex // 4
+    if what == "subnormal":  # weights, scales, errors and updates around 2^-126
+        W = torch.ldexp(W, torch.linspace(-140, -115, N).int().view(N, 1))
+    if what == "outliers":  # late columns grow past +-8 scales
+        W[:, ::7] *= 40
+        W[:, K - 64:] *= 1e-3
+    U = _factor(K, K, ex)
+    if what == "outliers":
+        U[:K - 64, K - 40:] *= 200
+    if what == "special":
+        W[1, 5], W[2, 70], W[3, K - 1] = float("nan"), float("inf"), -float("inf")
+        W[4] = 0
+        W[5, :64] = 0
+    Wq, S = _run(k, W, U)
+    Wq_o, S_o, _ = O.gptq(W.numpy(), U.numpy(), 128)
+    assert np.array_equal(S, S_o)
+    assert np.array_equal(Wq, Wq_o)
+
+
 def test_quantize_layer_beats_round_to_nearest(k):
     """End to end on the GPU (Hessian, factor, kernels): the layer's output error on the
     calibration data is well below round to nearest's, through ns_w4_linear."""
