@@ -759,7 +759,8 @@ __global__ __launch_bounds__(NWN * KS * kWave, BM >= 256 && KS == 1 ? 2 : 1) voi
 // Epilogue of the 16x16x32 GEMMs: a wave's BM x 32 accumulators (16-row fragments i, 16-column
 // halves jj; registers r, r + 1 are rows m, m + 1 of one column) rounded to bf16 into its private
 // LDS sub-tile lds (row stride 32), then stored as 16-byte row segments of C (element by element
-// at the edges of C or when C's rows are not 16-byte aligned).
+// only where C's rows are not whole aligned segments: a tile that merely ends past row M stored
+// element by element takes 5 us longer, as long as the K loop at K = 640).
 template <int BM>
 __device__ __forceinline__ void store_tile_16x16(const f32x4_t (&acc)[BM / 16][2], uint16_t* lds,
                                                  uint16_t* C, int M, int N, int m0, int n0w, int lane) {
@@ -777,15 +778,14 @@ __device__ __forceinline__ void store_tile_16x16(const f32x4_t (&acc)[BM / 16][2
       }
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's sub-tile is in LDS
   const int cr = lane >> 2, cc = lane & 3;
-  const bool full = m0 + BM <= M && n0w + 32 <= N && (N & 7) == 0 &&
-                    (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+  const bool whole = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;  // segments
 #pragma unroll
   for (int p = 0; p < BM / 16; ++p) {
     const int row = 16 * p + cr;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * 32 + 8 * cc]);
     const int m = m0 + row, n = n0w + 8 * cc;
-    if (full) {
-      *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = v;
+    if (whole) {
+      if (m < M && n < N) *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = v;
     } else if (m < M) {
       for (int e = 0; e < 8; ++e)
         if (n + e < N) C[(size_t)m * N + n + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
@@ -798,8 +798,8 @@ __device__ __forceinline__ void store_tile_16x16(const f32x4_t (&acc)[BM / 16][2
 // column j of its 16-column half, so a gate value (j < 8) finds its up value in lane j + 8 of the
 // same row. Y[m][o] = bf16(silu(g) * u) with g, u rounded to bf16 first (the values the plain
 // GEMM would store), o = 8 b + j; the wave's 16 outputs per row go through its private LDS
-// sub-tile (row stride 16) and out as 16-byte segments (element by element at the edges of Y or
-// when its rows are not 16-byte aligned).
+// sub-tile (row stride 16) and out as 16-byte segments (element by element where Y's rows are not
+// whole aligned segments).
 template <int BM>
 __device__ __forceinline__ void store_tile_16x16_swiglu(const f32x4_t (&acc)[BM / 16][2], uint16_t* lds,
                                                         uint16_t* Y, int M, int N, int m0, int n0w,
@@ -818,8 +818,7 @@ __device__ __forceinline__ void store_tile_16x16_swiglu(const f32x4_t (&acc)[BM 
       }
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's sub-tile is in LDS
   const int o0 = n0w >> 1;             // the wave's first output column
-  const bool full = m0 + BM <= M && n0w + 32 <= N && (Nh & 7) == 0 &&
-                    (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
+  const bool whole = (Nh & 7) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;  // segments
   const int cr = lane >> 1, cc = lane & 1;
 #pragma unroll
   for (int p = 0; p < (BM + 31) / 32; ++p) {
@@ -827,8 +826,8 @@ __device__ __forceinline__ void store_tile_16x16_swiglu(const f32x4_t (&acc)[BM 
     if (BM % 32 != 0 && row >= BM) continue;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * 16 + 8 * cc]);
     const int m = m0 + row, o = o0 + 8 * cc;
-    if (full) {
-      *reinterpret_cast<u32x4_t*>(&Y[(size_t)m * Nh + o]) = v;
+    if (whole) {
+      if (m < M && o < Nh) *reinterpret_cast<u32x4_t*>(&Y[(size_t)m * Nh + o]) = v;
     } else if (m < M) {
       for (int e = 0; e < 8; ++e)
         if (2 * (o + e) < N) Y[(size_t)m * Nh + o + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
