@@ -758,9 +758,9 @@ __global__ __launch_bounds__(NWN * KS * kWave, BM >= 256 && KS == 1 ? 2 : 1) voi
 
 // Epilogue of the 16x16x32 GEMMs: a wave's BM x 32 accumulators (16-row fragments i, 16-column
 // halves jj; registers r, r + 1 are rows m, m + 1 of one column) rounded to bf16 into its private
-// LDS sub-tile lds (row stride 32), then stored as 16-byte row segments of C (element by element
-// only where C's rows are not whole aligned segments: a tile that merely ends past row M stored
-// element by element takes 5 us longer, as long as the K loop at K = 640).
+// LDS sub-tile lds (row stride 32), then stored as 16-byte row segments of C. Rows that are not whole
+// aligned segments go out element by element, consecutive lanes on consecutive columns; a tile that
+// merely ends past row M does not (it took 5 us longer, as long as the K loop at K = 640).
 template <int BM>
 __device__ __forceinline__ void store_tile_16x16(const f32x4_t (&acc)[BM / 16][2], uint16_t* lds,
                                                  uint16_t* C, int M, int N, int m0, int n0w, int lane) {
@@ -781,14 +781,15 @@ __device__ __forceinline__ void store_tile_16x16(const f32x4_t (&acc)[BM / 16][2
   const bool whole = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;  // segments
 #pragma unroll
   for (int p = 0; p < BM / 16; ++p) {
-    const int row = 16 * p + cr;
-    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * 32 + 8 * cc]);
-    const int m = m0 + row, n = n0w + 8 * cc;
+    const int m = m0 + 16 * p + cr, n = n0w + 8 * cc;
     if (whole) {
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[(16 * p + cr) * 32 + 8 * cc]);
       if (m < M && n < N) *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = v;
-    } else if (m < M) {
-      for (int e = 0; e < 8; ++e)
-        if (n + e < N) C[(size_t)m * N + n + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+    } else {  // two rows of 32 elements at a time
+      for (int e = 0; e < 16; e += 2) {
+        const int row = 16 * p + e + (lane >> 5), c = lane & 31;
+        if (m0 + row < M && n0w + c < N) C[(size_t)(m0 + row) * N + n0w + c] = lds[row * 32 + c];
+      }
     }
   }
 }
@@ -824,13 +825,13 @@ __device__ __forceinline__ void store_tile_16x16_swiglu(const f32x4_t (&acc)[BM 
   for (int p = 0; p < (BM + 31) / 32; ++p) {
     const int row = 32 * p + cr;
     if (BM % 32 != 0 && row >= BM) continue;
-    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * 16 + 8 * cc]);
     const int m = m0 + row, o = o0 + 8 * cc;
     if (whole) {
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * 16 + 8 * cc]);
       if (m < M && o < Nh) *reinterpret_cast<u32x4_t*>(&Y[(size_t)m * Nh + o]) = v;
     } else if (m < M) {
       for (int e = 0; e < 8; ++e)
-        if (2 * (o + e) < N) Y[(size_t)m * Nh + o + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+        if (o + e < Nh) Y[(size_t)m * Nh + o + e] = lds[row * 16 + 8 * cc + e];
     }
   }
 }

@@ -121,6 +121,37 @@ def test_packed_ragged(kernels, M, N, K):
         assert torch.equal(kernels.w4_linear_packed_swiglu(x, wp, sp, N), two)
 
 
+# rows that are no whole 16-byte segments (N % 8 != 0, or an output at another address), in each of the
+# packed GEMM's plans and at full and ragged tiles; the elements around the output stay as they are
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (64, 201, 128), (100, 897, 1024), (128, 8201, 1024), (77, 203, 256), (260, 4097, 128), (410, 3583, 2048),
+    (500, 4606, 256), (700, 3501, 384), (333, 8962, 256), (1000, 4610, 2048), (1210, 4607, 2176),
+    (1900, 4609, 128), (1153, 3585, 2048), (548, 9986, 256), (128, 4609, 256), (700, 4608, 384),
+    (1000, 4608, 2048), (1210, 4608, 2176), (260, 4096, 128)])
+def test_packed_rows_without_segments(kernels, M, N, K):
+    wq, s = _weights(N, K, 128, M + N)
+    wp, sp = kernels.w4_repack(wq, s)
+    x = _x(M, K, K)
+
+    def at(cols, off):
+        flat = torch.full((M * cols + 64,), 7.0, dtype=BF16, device="cuda")
+        return flat, flat[32 + off:32 + off + M * cols].view(M, cols)
+
+    flat, y = at(N, 1 if N % 8 == 0 else 0)
+    assert kernels.w4_linear_packed(x, wp, sp, N, out=y) is y
+    lo = (y.data_ptr() - flat.data_ptr()) // 2
+    assert bool((flat[:lo] == 7).all()) and bool((flat[lo + M * N:] == 7).all())
+    ref = x.double() @ _deq(wq, s, 128).to(BF16).double().t()
+    err = (y.double() - ref).abs()
+    assert bool((err <= ref.abs() * 2.0 ** -8 + 2e-5 * ref.abs().max()).all())
+    if N % 16 == 0:
+        flat, y = at(N // 2, 1)
+        kernels.w4_linear_packed_swiglu(x, wp, sp, N, out=y)
+        assert torch.equal(y, kernels.w4_linear_packed_swiglu(x, wp, sp, N))
+        assert bool((flat[:33] == 7).all()) and bool((flat[33 + M * N // 2:] == 7).all())
+
+
 def test_rows_entry_points_reject():
     from nanoserve_amd import Kernels
 
