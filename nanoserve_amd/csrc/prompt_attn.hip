@@ -264,10 +264,11 @@ __global__ void __launch_bounds__(256, 2) prompt_attn_kernel(AttnArgs a) {
       }
   };
 
-  // Block b is ready once every wave's loads of it have landed (its own wait, then the barrier),
-  // and past that barrier nobody reads block b - 1, whose stage takes block b + 1.
+  // Block b is ready once every wave's loads of it have landed, and past the barrier nobody reads block
+  // b - 1, whose stage takes block b + 1: each wave waits for its loads of b and its reads of b - 1.
   auto ready = [] {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
