@@ -339,9 +339,9 @@ __global__ void __launch_bounds__(256) prompt_attn_merge_kernel(AttnArgs a) {
 }
 
 // Splits over the keys: enough for one and a half workgroups per CU, each with at least four blocks.
-// us (28 / 4 heads) for 1, 1.5, 2 and 3 per CU: 512 tokens at 3000 59.3, 53.3, 61.2, 61.7; 2000 tokens
-// at 0 60.1, 60.1, 72.6, 71.2; 200 at 4000 41.9, 38.6, 44.1, 43.1. With two blocks or one at least,
-// 20 tokens at 4000 take 30 and 39 us against 23.5, 200 at 0 14.3 and 13.7 against 10.2.
+// us (28 / 4 heads) for 1, 1.5, 2 and 3 per CU: 512 tokens at 3000 67.5, 60.9, 68.4, 67.4; 2000 tokens
+// at 0 56.4, 56.3, 66.5, 66.0; 200 at 4000 45.8, 39.5, 46.3, 42.1. With two blocks or one at least,
+// 20 tokens at 4000 take 26.2 and 30.9 us against 23.1, 200 at 0 14.2 and 16.0 against 10.1.
 int attn_splits(int T, int Hq, int Hk, int pos0) {
   int cus = 256;  // the device's CU count (a failed query leaves MI355X's; the launch reports it)
   if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;

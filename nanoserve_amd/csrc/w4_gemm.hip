@@ -261,8 +261,8 @@ __global__ __launch_bounds__(NWN * kWave) void w4_gemm_kernel(
 // a BMW x WN sub-tile (rows m0 .., columns n0w ..): its 32x32 accumulators are rounded to
 // bf16 and written to a wave-private LDS tile of row stride LS elements with 2-byte stores
 // (LS = WN + 8, where it fits, keeps the two row halves of a store on different banks), then
-// read back 16 bytes per lane and stored to Y as whole 16-byte row segments. Rows past M /
-// columns past N are not stored.
+// read back 16 bytes per lane and stored to Y as whole 16-byte row segments. Rows past M are not
+// stored (N is a multiple of the tile's columns).
 template <int MI, int NJ, int LS>
 __device__ __forceinline__ void store_tile_lds(const f32x16_t (&acc)[MI][NJ], uint16_t* lds, uint16_t* C,
                                                int M, int N, int m0, int n0w) {
@@ -285,39 +285,13 @@ __device__ __forceinline__ void store_tile_lds(const f32x16_t (&acc)[MI][NJ], ui
   constexpr int CPR = WN / 8;          // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;        // rows per 64-lane pass
   const int cr = lane / CPR, cc = lane % CPR;
-  const bool full = m0 + BMW <= M && n0w + WN <= N;
 #pragma unroll
   for (int p = 0; p < BMW / RPI; ++p) {
     const int row = p * RPI + cr;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(&lds[row * LS + 8 * cc]);
     const int m = m0 + row, n = n0w + 8 * cc;
-    if (full || (m < M && n + 8 <= N)) {
-      *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = v;
-    } else if (m < M) {
-      for (int e = 0; e < 8; ++e)
-        if (n + e < N) C[(size_t)m * N + n + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-    }
+    if (m < M) *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = v;
   }
-}
-
-// Direct epilogue (used when the tile does not fit the LDS ring): one bf16 store per value.
-// D[i][j] of lane l, register r: j = l % 32, i = 8 (r / 4) + 4 (l / 32) + r % 4.
-template <int MI, int NJ>
-__device__ __forceinline__ void store_tile_direct(const f32x16_t (&acc)[MI][NJ], uint16_t* C, int M,
-                                                  int N, int m0, int n0w) {
-  const int lane = threadIdx.x & 63, ln = lane & 31, kh = lane >> 5;
-  const bool full = m0 + 32 * MI <= M && n0w + 32 * NJ <= N;
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int n = n0w + 32 * j + ln;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + 32 * i + 8 * (r >> 2) + 4 * kh + (r & 3);
-        if (full || (m < M && n < N)) C[(size_t)m * N + n] = (uint16_t)f32_to_bf16_rne(acc[i][j][r]);
-      }
-    }
 }
 
 // SwiGLU epilogue (weights' rows are gate and up rows interleaved in blocks of 8: columns 16b ..
@@ -375,14 +349,13 @@ __device__ __forceinline__ void wait_vmcnt_c() {
 
 // K-split handoff of the GEMMs: groups 1 .. KS-1 hand their accumulators (MI x NJ vectors of R
 // floats) to group 0 through the free LDS ring `lds` (FLOATS floats; group g's wave wv of NWN in
-// lane-major order: word r * 64 + lane of its slice), and group 0 adds them in group order. Where
-// the ring holds every group's accumulators at once they go in one round; otherwise one group per
-// round. Every wave of the workgroup calls it (it holds barriers).
+// lane-major order: word r * 64 + lane of its slice), which holds all of them at once, and group 0 adds
+// them in group order. Every wave of the workgroup calls it (it holds barriers).
 template <int KS, int NWN, int FLOATS, int MI, int NJ, typename V>
 __device__ __forceinline__ void k_group_handoff(V (&acc)[MI][NJ], float* lds, int wv, int ks, int lane) {
   constexpr int R = sizeof(V) / sizeof(float);
   constexpr int WAVE = kWave * MI * NJ * R;  // floats per wave
-  constexpr bool kOneRound = (KS - 1) * NWN * WAVE <= FLOATS;
+  static_assert((KS - 1) * NWN * WAVE <= FLOATS, "every handed group's accumulators fit the ring");
   float* pb = lds + wv * WAVE + lane;
   auto put = [&](float* p) {
 #pragma unroll
@@ -400,23 +373,13 @@ __device__ __forceinline__ void k_group_handoff(V (&acc)[MI][NJ], float* lds, in
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[i][j][r] += p[((i * NJ + j) * R + r) * kWave];
   };
-  if constexpr (kOneRound) {
-    if (ks > 0) put(pb + (ks - 1) * NWN * WAVE);
-    lds_sync();
-    if (ks == 0) {
+  if (ks > 0) put(pb + (ks - 1) * NWN * WAVE);
+  lds_sync();
+  if (ks == 0) {
 #pragma unroll 1
-      for (int g = 1; g < KS; ++g) add(pb + (g - 1) * NWN * WAVE);
-    }
-    lds_sync();  // group 0's waves have read their slices before the epilogue reuses the LDS
-  } else {
-#pragma unroll 1
-    for (int g = 1; g < KS; ++g) {
-      if (ks == g) put(pb);
-      lds_sync();
-      if (ks == 0) add(pb);
-      lds_sync();
-    }
+    for (int g = 1; g < KS; ++g) add(pb + (g - 1) * NWN * WAVE);
   }
+  lds_sync();  // group 0's waves have read their slices before the epilogue reuses the LDS
 }
 
 // K-split handoff with the epilogue shared: every group adds up and stores one KS-th of its tile's
@@ -489,8 +452,8 @@ __device__ __forceinline__ int part_row(int ks, int e) {
 }
 
 // Epilogue of one part of a wave's 32-column slice (k_group_share): E values per lane, rounded to
-// bf16, through the wave's LDS slot (row stride 32) and out as 16-byte row segments. Rows past M
-// and columns past N are not stored.
+// bf16, through the wave's LDS slot (row stride 32) and out as 16-byte row segments. Rows past M are
+// not stored (N is a multiple of the tile's columns).
 template <int E>
 __device__ __forceinline__ void store_part(const float (&v)[E], uint16_t* lds, uint16_t* C, int M, int N,
                                            int m0, int n0w, int ks, int lane) {
@@ -512,12 +475,7 @@ __device__ __forceinline__ void store_part(const float (&v)[E], uint16_t* lds, u
     const int m = m0 + (E >= 4 ? 2 * E * ks + row : part_row<E>(ks, 0) + 4 * (row >> 1) + (row & 1));
     if (row < 2 * E && m < M) {
       const u32x4_t t = *reinterpret_cast<const u32x4_t*>(&lds[row * 32 + 8 * (lane & 3)]);
-      if (n + 8 <= N) {
-        *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = t;
-      } else {
-        for (int c = 0; c < 8; ++c)
-          if (n + c < N) C[(size_t)m * N + n + c] = (uint16_t)(t[c >> 1] >> (16 * (c & 1)));
-      }
+      *reinterpret_cast<u32x4_t*>(&C[(size_t)m * N + n]) = t;
     }
   }
 }
@@ -559,7 +517,7 @@ __global__ __launch_bounds__(NWN * KS * kWave, BM >= 256 && KS == 1 ? 2 : 1) voi
   constexpr int PART = KS > 1 ? NWN * kWave * MI * NJ * 16 * 2 : 0;  // one group's partials
   __shared__ __align__(16) uint16_t As[RING > PART ? RING : PART];
   constexpr int ELS = NWN * BM * (WN + 8) <= RING ? WN + 8 : WN;  // epilogue row stride
-  constexpr bool kLdsEpilogue = NWN * BM * ELS <= RING;
+  static_assert(KS > 1 || NWN * BM * ELS <= RING, "the epilogue's sub-tiles fit the ring");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wq = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -750,10 +708,8 @@ __global__ __launch_bounds__(NWN * KS * kWave, BM >= 256 && KS == 1 ? 2 : 1) voi
       store_part<E>(own, reinterpret_cast<uint16_t*>(slot), C, M, N, m0, n0 + wv * WN, ks, lane);
   } else if constexpr (SW)
     store_tile_swiglu<MI, NJ>(acc, C, M, N, m0, n0 + wv * WN);
-  else if constexpr (kLdsEpilogue)
-    store_tile_lds<MI, NJ, ELS>(acc, &As[wv * BM * ELS], C, M, N, m0, n0 + wv * WN);
   else
-    store_tile_direct<MI, NJ>(acc, C, M, N, m0, n0 + wv * WN);
+    store_tile_lds<MI, NJ, ELS>(acc, &As[wv * BM * ELS], C, M, N, m0, n0 + wv * WN);
 }
 
 // Epilogue of the 16x16x32 GEMMs: a wave's BM x 32 accumulators (16-row fragments i, 16-column
@@ -1113,7 +1069,7 @@ constexpr TileCfg kCfgs[] = {
     {64, 64, 1.00f},    // 9: v2, BM 64, K split over 4 wave groups of 2, 2 stages, two per CU
     {32, 32, 1.00f},    // 10: v2, BM 32, K split over 8 waves, 4 stages, one per CU
     {32, 64, 1.00f},    // 11: v2, BM 32, K split over 4 wave groups of 2, 4 stages, two per CU
-    {64, 32, 1.00f},    // 12: v2, BM 64, K split over 4 waves, 4 stages, two per CU
+    {64, 32, 1.00f},    // 12: v2, BM 64, K split over 4 waves, 4 stages, one per CU
     {32, 64, 1.00f},    // 13: v2, BM 32, K split over 4 wave groups of 2, 3 stages, three per CU
     {64, 128, 1.00f},   // 14: v2, BM 64, K split over 2 wave groups of 4, 4 stages, two per CU
     {96, 64, 1.00f},    // 15: v2, BM 96, K split over 4 wave groups of 2, 2 stages, one per CU
@@ -1277,6 +1233,41 @@ hipError_t launch_gemm_packed(const uint16_t* A, const uint32_t* Wp, const uint1
                 : launch_gemm_packed_t<false>(A, Wp, Sp, C, M, N, K, plan, st);
 }
 
+namespace {
+// The pipelined kernel's plans, with either epilogue. WD: weights that many blocks ahead.
+template <bool SW>
+hipError_t launch_gemm2(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
+  const dim3 grid((a.N + p.bn - 1) / p.bn, (a.M + p.bm - 1) / p.bm);
+#define NS_GEMM2_CASE(P, BM, NWN, ST, KS, WD)                                                            \
+  case P:                                                                                                \
+    static_assert(kCfgs[P].bm == BM && kCfgs[P].bn == 32 * NWN, "tile of the plan");                     \
+    hipLaunchKernelGGL((w4_gemm2_kernel<BM, 32, NWN, ST, SW, KS, WD>), grid, dim3(64 * NWN * KS), 0, st, \
+                       a.A, a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));                                  \
+    return hipSuccess;
+  switch (p.cfg) {
+    NS_GEMM2_CASE(4, 128, 4, 3, 1, kWeightAhead)
+    NS_GEMM2_CASE(5, 128, 4, 2, 2, kWeightAhead)
+    NS_GEMM2_CASE(6, 256, 4, 2, 1, kWeightAhead)
+    NS_GEMM2_CASE(7, 256, 4, 2, 2, kWeightAhead)
+    NS_GEMM2_CASE(8, 128, 2, 2, 4, kWeightAhead)
+    NS_GEMM2_CASE(9, 64, 2, 2, 4, kWeightAhead)
+    NS_GEMM2_CASE(10, 32, 1, 4, 8, 1)
+    NS_GEMM2_CASE(11, 32, 2, 4, 4, 1)
+    NS_GEMM2_CASE(12, 64, 1, 4, 4, 1)
+    NS_GEMM2_CASE(13, 32, 2, 3, 4, 1)
+    NS_GEMM2_CASE(14, 64, 4, 4, 2, 1)
+    NS_GEMM2_CASE(15, 96, 2, 2, 4, kWeightAhead)
+    NS_GEMM2_CASE(16, 64, 4, 2, 2, kWeightAhead)
+    NS_GEMM2_CASE(17, 96, 4, 2, 2, kWeightAhead)
+    NS_GEMM2_CASE(18, 160, 4, 2, 2, kWeightAhead)
+    NS_GEMM2_CASE(19, 192, 4, 2, 2, kWeightAhead)
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef NS_GEMM2_CASE
+}
+}  // namespace
+
 hipError_t launch_gemm(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
   const dim3 grid((a.N + p.bn - 1) / p.bn, (a.M + p.bm - 1) / p.bm);
   switch (p.cfg) {
@@ -1292,145 +1283,13 @@ hipError_t launch_gemm(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
       hipLaunchKernelGGL((w4_gemm_kernel<128, 32, 4>), grid, dim3(256), 0, st, a.A, a.Wq, a.S,
                          a.C, a.M, a.N, a.K, a.G);
       return hipSuccess;
-    case 4:
-      hipLaunchKernelGGL((w4_gemm2_kernel<128, 32, 4, 3, false, 1, kWeightAhead>), grid, dim3(256), 0, st, a.A, a.Wq, a.S,
-                         a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 5:
-      hipLaunchKernelGGL((w4_gemm2_kernel<128, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 6:
-      hipLaunchKernelGGL((w4_gemm2_kernel<256, 32, 4, 2, false, 1, kWeightAhead>), grid, dim3(256), 0, st, a.A, a.Wq, a.S,
-                         a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 7:
-      hipLaunchKernelGGL((w4_gemm2_kernel<256, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq, a.S,
-                         a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 8:
-      hipLaunchKernelGGL((w4_gemm2_kernel<128, 32, 2, 2, false, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 9:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 2, 2, false, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 10:
-      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 1, 4, false, 8>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 11:
-      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 4, false, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 12:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 1, 4, false, 4>), grid, dim3(256), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 13:
-      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 3, false, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 14:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 4, false, 2>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 15:
-      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 2, 2, false, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 16:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 17:
-      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 18:
-      hipLaunchKernelGGL((w4_gemm2_kernel<160, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 19:
-      hipLaunchKernelGGL((w4_gemm2_kernel<192, 32, 4, 2, false, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
     default:
-      return hipErrorInvalidValue;
+      return launch_gemm2<false>(a, p, st);
   }
 }
 
 hipError_t launch_gemm_swiglu(const GemmArgs& a, const GemmPlan& p, hipStream_t st) {
-  const dim3 grid((a.N + p.bn - 1) / p.bn, (a.M + p.bm - 1) / p.bm);
-  switch (p.cfg) {
-    case 4:
-      hipLaunchKernelGGL((w4_gemm2_kernel<128, 32, 4, 3, true, 1, kWeightAhead>), grid, dim3(256), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 5:
-      hipLaunchKernelGGL((w4_gemm2_kernel<128, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 6:
-      hipLaunchKernelGGL((w4_gemm2_kernel<256, 32, 4, 2, true, 1, kWeightAhead>), grid, dim3(256), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 7:
-      hipLaunchKernelGGL((w4_gemm2_kernel<256, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 8:
-      hipLaunchKernelGGL((w4_gemm2_kernel<128, 32, 2, 2, true, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 9:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 2, 2, true, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A, a.Wq,
-                         a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 10:
-      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 1, 4, true, 8>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 11:
-      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 4, true, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 12:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 1, 4, true, 4>), grid, dim3(256), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 13:
-      hipLaunchKernelGGL((w4_gemm2_kernel<32, 32, 2, 3, true, 4>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 14:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 4, true, 2>), grid, dim3(512), 0, st, a.A, a.Wq, a.S, a.C,
-                         a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 15:
-      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 2, 2, true, 4, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 16:
-      hipLaunchKernelGGL((w4_gemm2_kernel<64, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 17:
-      hipLaunchKernelGGL((w4_gemm2_kernel<96, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 18:
-      hipLaunchKernelGGL((w4_gemm2_kernel<160, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    case 19:
-      hipLaunchKernelGGL((w4_gemm2_kernel<192, 32, 4, 2, true, 2, kWeightAhead>), grid, dim3(512), 0, st, a.A,
-                         a.Wq, a.S, a.C, a.M, a.N, a.K, ilog2(a.G));
-      return hipSuccess;
-    default:
-      return hipErrorInvalidValue;
-  }
+  return launch_gemm2<true>(a, p, st);
 }
 
 }  // namespace ns
