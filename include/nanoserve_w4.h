@@ -139,7 +139,7 @@ int ns_w4_linear_swiglu(const void* X, const void* Wq, const void* S, void* Y, i
                         int K, int G, void* stream);
 
 /*
- * Bytes of fp32 workspace ns_w4_gptq needs for N rows (128 * N * 4); 0 for N <= 0.
+ * Bytes of workspace ns_w4_gptq asks for with N rows (128 * N * 4); 0 for N <= 0.
  */
 size_t ns_w4_gptq_workspace(int N);
 
@@ -150,7 +150,8 @@ size_t ns_w4_gptq_workspace(int N);
  *   W [N][K] fp32: the weights, overwritten (working memory; its contents afterwards are
  *   unspecified). U [K][K] fp32: the upper Cholesky factor of the damped inverse Hessian of the
  *   layer's calibration activations (U^T U = (2 X^T X / T + damping)^-1), computed by the caller;
- *   only its upper triangle is read. work: ns_w4_gptq_workspace(N) bytes of device memory.
+ *   only its upper triangle is read. work: ns_w4_gptq_workspace(N) bytes of device memory
+ *   (required and checked; the kernels keep their errors in W and do not touch it).
  * Column i of each row is quantized with the round-to-nearest rule of ns_w4_quantize, the group
  * scale taken from the row's group values as they stand when the group starts; its error
  * e = (w_i - (q - 8) s) / U[i][i] updates each later column j as w_j <- fma(-e, U[i][j], w_j),

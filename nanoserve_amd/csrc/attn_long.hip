@@ -4,8 +4,9 @@
 //
 // Bound by HBM. decode_attn_kernel gives each 128 cache rows two workgroups that load everything at
 // once and end; over a long cache that is rounds of short-lived workgroups, each reading the K rows
-// twice, preparing q and leaving partials for every 128 rows. Here about one eight-wave workgroup per
-// CU streams a contiguous range of rows:
+// twice, preparing q and leaving partials for every 128 rows. Here at most one eight-wave workgroup per
+// CU streams a contiguous range of rows (whole multiples of 128, so just past a multiple of the launch's
+// workgroups fewer of them have rows: 8320 rows of 4 kv heads keep 132 of 256 busy):
 //  * Each wave takes every eighth 16-row block of the range through its own two-stage LDS ring
 //    (8 KiB of K and V per stage by coalesced buffer-to-LDS loads, 128 KiB per workgroup), waiting
 //    only for its own loads: no barrier in the loop, 64 KiB and more in flight per CU.
@@ -15,7 +16,8 @@
 //    (rows 4 (l / 16) .. + 3 of one dimension per lane) is one ds_read_b64_tr_b16 per 16 dimensions.
 //  * The workgroups' results are merged by decode_attn_merge_kernel.
 // Rows per workgroup come from the position (long_chunk_rows), so that a short conversation in a
-// large cache still spreads over workgroups of 128 rows.
+// large cache still spreads over workgroups of 128 rows (28 / 4 heads, 32768 rows, position 1000: 24.0
+// -> 10.3 us with the merge).
 #include <math.h>
 #include <stdint.h>
 
@@ -330,7 +332,7 @@ __global__ void __launch_bounds__(kWaves * kWave) attn_long_kernel(LongArgs a) {
 
 }  // namespace
 
-// About one workgroup per CU; never more splits than 128-row pieces of the cache (the workspace).
+// At most one workgroup per CU; never more splits than 128-row pieces of the cache (the workspace).
 int attn_long_splits(int Hk, int max_len) {
   int cus = 256;
   if (cached_cu_count(&cus) != hipSuccess || cus <= 0) cus = 256;

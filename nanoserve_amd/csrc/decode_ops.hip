@@ -755,7 +755,9 @@ int attn_check(int Hq, int Hk, int D, int max_len, size_t work_bytes, const void
 // Caches whose 128-row pieces of all kv heads outnumber the CUs are streamed (attn_long.hip), if the
 // launch merges. Either side of that line on MI355X, us with the merge (28 / 4, 12 / 2, 32 / 8 heads;
 // decode_attn_kernel first): 256 pieces 11.2 / 11.9, 11.6 / 12.0, 11.2 / 11.3; 512 pieces 16.8 / 14.5,
-// 18.6 / 14.7, 15.4 / 14.0.
+// 18.6 / 14.7, 15.4 / 14.0. Just above the line, where ranges of whole pieces keep only half of the
+// streaming workgroups busy, it is ahead too: 28 / 4 heads 260 pieces 13.8 / 12.5, 320 13.8 / 13.1, 384
+// 14.6 / 13.7, 516 20.2 / 15.4; 12 / 2 heads 258 15.1 / 12.5, 314 16.4 / 12.9; 32 / 8 heads 520 18.0 / 15.1.
 template <bool kFused>
 int launch_attn(const void* q, const void* bias, const void* inv_freq, void* kc, void* vc,
                 const int* pos, void* out, void* work, int Hq, int Hk, int max_len,

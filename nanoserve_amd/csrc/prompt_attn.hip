@@ -16,9 +16,9 @@ namespace {
 
 // ------------------------------------------------------------------ bias + RoPE + KV append
 // Bound by launch and memory latency (1000 tokens of 36 heads: 9.5 us with the KV append, where
-// separate bias, RoPE and cache-copy launches took about 60). Thread (token, head block, chunk c) rotates elements 8c ..
-// 8c + 7 with their partners D/2 further on in up to kQkvHeads heads, so the eight sincosf of a
-// chunk serve all of them and 2 kQkvHeads 16-byte loads are in flight per thread.
+// separate bias, RoPE and cache-copy launches took about 60). Thread (token, head block, chunk c)
+// rotates elements 8c .. 8c + 7 with their partners D/2 further on in up to kQkvHeads heads, so the
+// eight sincosf of a chunk serve all of them and 2 kQkvHeads 16-byte loads are in flight per thread.
 constexpr int kQkvHeads = 6;
 __global__ void __launch_bounds__(256)
     prompt_qkv_kernel(uint16_t* __restrict__ qkv, const uint16_t* __restrict__ bias,
@@ -100,16 +100,16 @@ __global__ void __launch_bounds__(256)
 //    leave (exact in fp32). Prompts from position 0 take two (16 significant bits, where fused bf16
 //    attention holds 8). Chunks after cached positions take three, the whole fp32 probability, as an
 //    attention in fp32 holds it: with two, 0.23 % of the outputs are not the rounding of the float64
-//    result, with three 0.04 %, for fp32 SDPA 0.07 % (28 / 4 heads, 512 tokens at 3000; 62.6 us
-//    against 54.9 with two).
+//    result, with three 0.04 %, for fp32 SDPA 0.07 % (28 / 4 heads, 512 tokens at 3000; 61.1 us
+//    against 53.6 with two).
 //  * LDS rows are 256 B (16 chunks of 16 B): K chunks are XOR-swizzled by row % 16 (the 16 rows of
 //    a fragment read hit distinct banks), V chunks by 4 (row % 4) (the 4-row x 64 B transpose
 //    reads spread over all banks).
-// MI355X, 28 / 4 heads: 1000 tokens from position 0 35.6 us with the merge (PyTorch's fused SDPA on repeated
-// K / V 67 us and its copies 40); 512 tokens after 3000 cached ones 62.6 us (fp32 SDPA 682 us and its
-// copies 60).
 //  * Few row tiles (short prompts, few kv heads) leave CUs idle: the keys are then split over
 //    blockIdx.z and a second kernel merges the fp32 partials.
+// MI355X, 28 / 4 heads, with the merge: 1000 tokens from position 0 36.1 us (PyTorch's fused SDPA on
+// repeated K / V 67 us and its copies 40); 512 tokens after 3000 cached ones 60.9 us (fp32 SDPA 682
+// us and its copies 60).
 constexpr int kD = 128;
 constexpr int kRows = 128;    // query rows per workgroup
 constexpr int kKeys = 64;     // keys per block

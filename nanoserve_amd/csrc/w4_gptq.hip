@@ -20,8 +20,11 @@
 // group needs the errors E of the group before it):
 //  * panel workgroups bring the group's own 128 columns up to date with the errors of group
 //    g - 1, quantize them column after column and write codes, scales and the errors of group g;
-//  * trailing workgroups apply the errors of group g - 1 to every column after group g. They fill
-//    the chip while the panel, a serial chain per row, would leave it idle.
+//  * trailing workgroups apply the errors of group g - 1 to every column after group g, on the CUs
+//    that the panels, a serial chain per row, leave with little to do.
+// 4608 x 3584 on MI355X: a launch of panels alone takes 26.7 us, the one with 936 trailing tiles 60.8
+// (25.8 us of fp32 matrix work), all 28 launches 1.2 ms without gaps. The trailing work runs close to
+// its rate, but the panels' chain adds to it.
 // E lives where it is no longer needed: error i of row n replaces W[n][k0 + i].
 //
 // Both rank-128 updates run on the fp32 matrix cores. v_mfma_f32_32x32x2_f32 and

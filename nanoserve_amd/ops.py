@@ -72,8 +72,9 @@ else:  # pragma: no cover - older torch builds
         return torch.cuda.current_stream(device).cuda_stream
 
 
-# The current device index without torch.cuda.current_device()'s initialisation check: every caller
-# has a GPU tensor in hand, so the runtime is initialised.
+# The current device index without torch.cuda.current_device()'s initialisation check: the callers have
+# GPU tensors in hand (and reading the raw stream, as probe_empty does without any, initialises the
+# runtime itself).
 _current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
@@ -195,7 +196,8 @@ class Kernels:
         the next step): W [N, K] (any float dtype) and U [K, K] fp32, the upper Cholesky factor
         of the layer's damped inverse Hessian (``nanoserve_amd.gptq.hessian_factor``) ->
         (Wq int32 [N, K // 8], S bf16 [N, K // group]) in w4_quantize's format. W is not
-        modified (the kernels work on an fp32 copy)."""
+        modified (the kernels work on an fp32 copy; the workspace is the entry point's contract,
+        they do not use it)."""
         if not isinstance(W, torch.Tensor) or not W.is_cuda:
             raise ValueError("W must be a CUDA (HIP) tensor")
         _require_gpu_tensor(U, "U", torch.float32)
@@ -224,11 +226,11 @@ class Kernels:
         """x [M, K] bf16 -> y [M, N] bf16 = x @ deq(Wq, S)^T. Reference ops.py:85-97.
 
         Any M runs natively (the reference pads 3 -> 4 and 5..7 -> 8 with zero rows, and larger M
-        up to a multiple of 128, which does not change any output row). ``out`` (not in the reference): a contiguous [M, N]
-        bf16 tensor to write instead of a new one, for M <= 8 and multiples of 128 (the M the reference does not pad). ``work`` (not in
-        the reference): a workspace from ``w4_linear_workspace``; with it the M = 2..8 GEMV
-        may split long rows over K (ns_w4_linear_ws), without it no shape is split
-        (ns_w4_linear)."""
+        up to a multiple of 128, which does not change any output row). ``out`` (not in the
+        reference): a contiguous [M, N] bf16 tensor to write instead of a new one, for M <= 8 and
+        multiples of 128 (the M the reference does not pad). ``work`` (not in the reference): a
+        workspace from ``w4_linear_workspace``; with it the M = 2..8 GEMV may split long rows over
+        K (ns_w4_linear_ws), without it no shape is split (ns_w4_linear)."""
         _require_gpu_tensor(x, "x", torch.bfloat16)
         _require_gpu_tensor(Wq, "Wq", torch.int32)
         _require_gpu_tensor(S, "S", torch.bfloat16)

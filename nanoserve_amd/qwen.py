@@ -21,11 +21,12 @@ Kernels used per decode step and layer: ns_w4_gemv_decode x3 (the q/k/v and gate
 with the residual add + RMSNorm fused into their activation load, SwiGLU fused into the
 gate/up GEMV's output; the down GEMV), ns_decode_qkv_attention (bias + RoPE + KV append +
 grouped-query attention over the cache, splits left unmerged) and ns_w4_gemv_decode_attn
-(the o GEMV, merging the attention's splits while loading its activation). The gate/up weight rows are stored interleaved in blocks of 8
-(``interleave_gate_up``) so that a gate row and its up row land in the same 16-row group. The prompt pass (T > 1) uses ns_w4_linear (GEMM for T > 8) and ns_w4_linear_swiglu,
-ns_rmsnorm, ns_prompt_qkv (bias + RoPE + KV append) and ns_prompt_attention (causal attention on
-matrix cores; PyTorch SDPA for head sizes other than 128); after
-``pack_prefill`` prompts of more than 16 tokens run the packed-format GEMMs instead
+(the o GEMV, merging the attention's splits while loading its activation). The gate/up weight
+rows are stored interleaved in blocks of 8 (``interleave_gate_up``) so that a gate row and its
+up row land in the same 16-row group. The prompt pass (T > 1) uses ns_w4_linear (GEMM for
+T > 8) and ns_w4_linear_swiglu, ns_rmsnorm, ns_prompt_qkv (bias + RoPE + KV append) and
+ns_prompt_attention (causal attention on matrix cores; PyTorch SDPA for head sizes other than
+128); after ``pack_prefill`` prompts of more than 16 tokens run the packed-format GEMMs instead
 (ns_w4_linear_packed, ns_w4_linear_packed_swiglu).
 
 No weights are downloaded: ``random`` builds a model of any Qwen2 shape with seeded random
