@@ -155,6 +155,29 @@ def test_prompt_ops_reject_bad_arguments():
     assert qkv(P, P + 2, P, P, P, 4, 4, 2, 128, 0, 16, None) == -2
 
 
+# past the position where the projection's row stride would end the 32-bit offsets, and the last one a
+# cache's rows reach: keys planted at the start, the middle and the end decide the result
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,pos0", [(70, 300000), (40, (1 << 23) - 169)])
+def test_prompt_attention_far_positions(kernels, T, pos0):
+    n, Hq = pos0 + T, 2
+    assert kernels.prompt_attention_fits(T, Hq, 1, pos0, 128)
+    assert T > 40 or not kernels.prompt_attention_fits(T, Hq, 1, pos0 + 1, 128)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    k, v = (torch.randn(1, n, 128, generator=g, device="cuda", dtype=BF16) for _ in range(2))
+    k *= 0.05
+    q = torch.randn(T, Hq * 128, generator=g, device="cuda").to(BF16)
+    q[:, ::128] = 16.0
+    for j in (5, n // 2, n - T - 1, n - 2):
+        k[0, j, 0] = 18.0
+    work = kernels.prompt_attention_workspace(T, Hq, 1, pos0)
+    got = kernels.prompt_attention(q, k, v, Hq, pos0, work=work).double().view(T, Hq, 128)
+    for h in range(Hq):
+        want = _ref(q.double().view(T, Hq, 128)[:, h:h + 1], k.double(), v.double(), pos0)
+        err = (got[:, h] - want).abs()
+        assert bool((err <= want.abs() * 2.0 ** -8 + 2.0 ** -14 * v.double().abs().amax()).all())
+
+
 def test_prompt_attention_limits_follow_the_key_rows():
     """The runner's choice of the kernel is the kernel's own rule: 32-bit offsets over the rows the keys
     lie in (128 values in a cache, the projection's width without one) and 65535 row tiles."""
